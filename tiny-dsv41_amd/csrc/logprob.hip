@@ -8,31 +8,48 @@
 // log-probs are given.
 //
 // The contraction is computed transposed, C^T[v, n] = sum_k w[v, k] x[n, k], so that an
-// MFMA lane owns one token column and the per-token softmax state lives in registers:
-// each lane of a 32x32 output block holds 16 vocabulary rows of one token.  A workgroup
-// owns BT = 256 tokens and sweeps a range of the vocabulary in BV = 256-row blocks (each
-// of its eight waves, two per SIMD, computes a 128 x 64 part); after each block the fp32
+// MFMA lane owns one token column and the per-token softmax state lives in registers.  A
+// workgroup owns BT = 256 tokens and sweeps a range of the vocabulary in BV = 256-row blocks
+// (each of its eight waves, two per SIMD, computes a 128 x 64 part); after each block the fp32
 // accumulators update a running (max, sum e, sum e*z) per token.  A second kernel merges
 // the vocabulary ranges and computes the target logit as its own dot product.
 //
+// Long runs are bound by the power limit: the multiplies' own energy sets the clock.  16x16x32
+// MFMAs were chosen for that (a loop of them alone over random bf16 operands runs at 2.00
+// PFLOP/s on this card, one of 32x32x16 at 1.75: half the accumulator traffic per operation).
+//
 // Operands move from HBM to LDS with buffer loads that write LDS directly (no register
 // staging), into two stage buffers of 64 hidden elements per row: 128 bytes, one whole
-// cache line of every row, so each line crosses L2 -> L1 once (with half-line stages
-// every line crosses twice, as the L1 cannot keep the other half until the next stage).
-// The stage sequence runs straight across vocabulary blocks, so the pipeline never
-// drains between blocks.  Each stage has one barrier, after its third k-step: before it
-// every wave waits for its own fragment reads of the stage and its own loads of the next
-// stage, so after it the next stage is readable by all and the current stage's buffer
-// takes the loads of the stage after next, a whole stage ahead of their use.  Those loads
-// and the next stage's first fragment reads are slotted between the multiplies of the
-// last k-step; the other k-steps carry the fragment reads of the k-step after them.  MFMA
-// operand fragments alternate between two register sets, so reads never wait for the
-// multiplies that use the other set.  Each 128-byte LDS row holds its eight 16-byte
-// chunks XOR-swizzled by (row >> 1) & 7; with that, a wave-wide 16-byte read of one chunk
-// of 32 consecutive rows is free of bank conflicts on gfx950's LDS (measured: 4 cycles per
-// read, against 8 for row & 7 and 32 unswizzled).
+// cache line of every row, so each line crosses L2 -> L1 once.  The stage sequence runs
+// straight across vocabulary blocks, so the pipeline never drains between blocks.
+//
+// The two waves of a SIMD work in turns.  A stage has four phases, one per quarter of the
+// wave's tile (64 weight rows x 32 tokens over the whole stage: 16 MFMAs, 256 cycles), and a
+// phase two parts with a barrier behind each: the first reads the quarter's fragments and
+// issues two loads, the second multiplies.  Waves 4-7 start one barrier late, so on every SIMD
+// one wave multiplies while the other reads, and the matrix core passes from one to the other
+// at each barrier.  (With one barrier per stage and reads between the multiplies of both
+// waves, one wave ran ahead and idled at the barrier while the other finished alone below the
+// MFMA rate: matrix cores busy 75% of the cycles, now 85%.  16384 x 7168 -> 129280, on one
+// box: 22.4 ms before, 22.7 with the turns and 32x32x16, where the clock fell as the cores
+// filled, 20.4 with the turns and 16x16x32; 8192 x 2048 -> 151936: 4.02, 3.65, 3.41 ms.)
+//
+// A quarter's rows are a region of the stage buffer (A0, A1, B0, B1: the halves of the weight
+// and of the token rows).  A region is reloaded as soon as its reads are over, not the stage:
+//   read in phase        B0(s) end of 4s-1, A0(s) 4s, B1(s) 4s+1, A1(s) 4s+2 (read = its
+//                        fragments back before the multiplies of 4s, 4s, 4s+1, 4s+2 end)
+//   loaded for s+2 in    B0 4s+2, A0 4s+3, B1 4s+4, A1 4s+5
+// so every load is in flight for four to five phases (about 2500 cycles), and each wave waits
+// in every phase only until all but its last LOADS_AHEAD = 8 loads (four phases' worth) have
+// landed, one barrier before the first wave reads them.
+//
+// Each 128-byte LDS row holds its eight 16-byte chunks XOR-swizzled by (row >> 1) & 7; with
+// that, a wave-wide 16-byte read of four chunks of 16 consecutive rows is free of bank
+// conflicts on gfx950's LDS (4 cycles per read, against 8 for row & 7 and 32 unswizzled).
 
 #include <math.h>
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -43,24 +60,24 @@ constexpr int WAVES_V = 2;                   // waves along the vocabulary
 constexpr int WAVES_T = 4;                   // waves along tokens
 constexpr int NWAVES = WAVES_V * WAVES_T;
 constexpr int NT = 64 * NWAVES;              // 8 waves, two per SIMD
-constexpr int WV = 4;                        // 32-row MFMA blocks per wave along the vocabulary
-constexpr int WT = 2;                        // 32-column MFMA blocks per wave along tokens
-constexpr int BV = WAVES_V * WV * 32;        // 256 vocabulary rows per block
-constexpr int BT = WAVES_T * WT * 32;        // 256 tokens per workgroup
+constexpr int WV = 8;                        // 16-row MFMA blocks per wave along the vocabulary
+constexpr int WT = 4;                        // 16-column MFMA blocks per wave along tokens
+constexpr int BV = WAVES_V * WV * 16;        // 256 vocabulary rows per block
+constexpr int BT = WAVES_T * WT * 16;        // 256 tokens per workgroup
 constexpr int BK = 64;                       // hidden elements per stage
-constexpr int KS = BK / 16;                  // MFMA k-steps per stage
+constexpr int KS = BK / 32;                  // MFMA k-steps per stage
 constexpr int ROWB = BK * 2;                 // bytes per LDS row: one 128-byte cache line
 constexpr int STAGE_BYTES = (BV + BT) * ROWB;  // 64 KiB
 constexpr int LDS_BYTES = 2 * STAGE_BYTES;   // two stage buffers
-constexpr int ROWS_PER_LOAD = 1024 / ROWB;   // rows one wave-wide 16-byte LDS load fills
-constexpr int A_LOADS = BV / NWAVES / ROWS_PER_LOAD;  // per wave per stage
-constexpr int B_LOADS = BT / NWAVES / ROWS_PER_LOAD;
+constexpr int A0 = 0, A1 = 1, B0 = 2, B1 = 3;  // a stage's regions: 128 weight or token rows each
+constexpr int REGION_BYTES = 128 * ROWB;
+constexpr int LOADS_AHEAD = 8;               // loads a wave keeps in flight past each wait
 constexpr int CU_COUNT = 256;                // MI355X
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float NEG_INF = -__builtin_huge_valf();
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
@@ -85,8 +102,10 @@ struct Params {
   int vbeg;
 };
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
+// Raw buffer descriptor: stride 0, reads at or past `bytes` return 0.
+__device__ __forceinline__ v4i rsrc(const void* base, uint32_t bytes) {
+  const uint64_t a = (uint64_t)(uintptr_t)base;
+  return v4i{(int)(uint32_t)a, (int)((uint32_t)(a >> 32) & 0xFFFFu), (int)bytes, 0x00020000};
 }
 
 // merge two softmax states (max, sum e, sum e*z)
@@ -123,52 +142,49 @@ __device__ __forceinline__ void block_coords(const Params& p, int b, int& tb, in
 // row % 16, so every 32-row MFMA block shares one pattern.
 __device__ __forceinline__ int swz(int row) { return (row >> 1) & 7; }
 
-// s_waitcnt vmcnt(0), expcnt and lgkmcnt left at their maxima: this wave's LDS loads landed.
-__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
-
-// Workgroup barrier with no memory fence: completion of the LDS loads is tracked with
-// wait_loads, and the memory clobber keeps the compiler from moving LDS accesses across.
-__device__ __forceinline__ void barrier() { asm volatile("s_barrier" ::: "memory"); }
-
-__device__ __forceinline__ void read_frags(const unsigned char* stage, int addr_a, int addr_b, bf16x8 (&fa)[WV],
-                                           bf16x8 (&fb)[WT]) {
-#pragma unroll
-  for (int i = 0; i < WV; ++i) fa[i] = *reinterpret_cast<const bf16x8*>(stage + addr_a + i * 32 * ROWB);
-#pragma unroll
-  for (int j = 0; j < WT; ++j) fb[j] = *reinterpret_cast<const bf16x8*>(stage + addr_b + j * 32 * ROWB);
+// Workgroup barrier with no memory fence: reads and loads of the LDS are ordered by the
+// phases (see fused_kernel); the memory clobber keeps the compiler from moving LDS accesses
+// across, the scheduling barriers keep the multiplies on their side.
+__device__ __forceinline__ void barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
 }
 
-// One k-step of the wave's WV x WT block of 32x32 outputs, with other work slotted
-// between the multiplies: after multiply i,
-// extra(i) issues one fragment read or load (each group is fenced so the scheduler
-// keeps the interleave).
-template <class Extra>
-__device__ __forceinline__ void mfma_set_x(floatx16 (&acc)[WV][WT], const bf16x8 (&fa)[WV], const bf16x8 (&fb)[WT],
-                                           Extra&& extra) {
-#pragma unroll
-  for (int i = 0; i < WV; ++i)
-#pragma unroll
-    for (int j = 0; j < WT; ++j) {
-      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
-      extra(i * WT + j);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+// One wave-wide load of 64 x 16 bytes straight to LDS (lane l to lds_addr + 16 l).  Written as
+// asm because the compiler otherwise waits for every load in flight before each LDS read; it
+// writes no register, and the phases wait for it by count (wait_loads).
+__device__ __forceinline__ void load_lds(v4i rs, uint32_t voff, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs),
+               "s"(lds_addr)
+               : "memory");
 }
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// e^(x ln 2): v_exp_f32 alone.  exp2f adds a rescue for results below 2^-126, which no sum
+// here can notice (the largest term of each is 1).
+__device__ __forceinline__ float exp2_raw(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// Vocabulary row of block i, accumulator register r, and token column of block j, relative to
+// the lane's first ones: a wave holds rows [64 wv, +64) and tokens [32 wt, +32) of both halves
+// of the workgroup's tile, a lane rows 4 (lane / 16) + r of each block and token lane % 16.
+constexpr int row_off(int i, int r) { return (i / 4) * (BV / 2) + (i % 4) * 16 + r; }
+constexpr int col_off(int j) { return (j / 2) * (BT / 2) + (j % 2) * 16; }
 
 // Folds one vocabulary block into the running (max z, sum e, sum e*z) of token column j.
 // Rows at offsets >= lim lie past the vocabulary (their weights read as zero) and are
 // skipped when MASK is set.
 template <bool MASK>
-__device__ __forceinline__ void absorb(const floatx16 (&acc)[WV][WT], int j, int lim, float invT, float& m,
+__device__ __forceinline__ void absorb(const floatx4 (&acc)[WV][WT], int j, int lim, float invT, float& m,
                                        float& s, float& a) {
   float mx = NEG_INF;
 #pragma unroll
   for (int i = 0; i < WV; ++i)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int off = i * 32 + 8 * (r >> 2) + (r & 3);
-      mx = fmaxf(mx, (!MASK || off < lim) ? acc[i][j][r] : NEG_INF);
-    }
+    for (int r = 0; r < 4; ++r) mx = fmaxf(mx, (!MASK || row_off(i, r) < lim) ? acc[i][j][r] : NEG_INF);
   const float mn = fmaxf(m, mx * invT);  // invT > 0: the max commutes with the scaling
   if (mn == NEG_INF) return;
   const float c1 = invT * LOG2E, mb = mn * LOG2E;
@@ -176,14 +192,13 @@ __device__ __forceinline__ void absorb(const floatx16 (&acc)[WV][WT], int j, int
 #pragma unroll
   for (int i = 0; i < WV; ++i)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int off = i * 32 + 8 * (r >> 2) + (r & 3);
+    for (int r = 0; r < 4; ++r) {
       const float v = acc[i][j][r];
-      const float e = exp2f((!MASK || off < lim) ? __builtin_fmaf(v, c1, -mb) : NEG_INF);
+      const float e = exp2_raw((!MASK || row_off(i, r) < lim) ? __builtin_fmaf(v, c1, -mb) : NEG_INF);
       sum += e;
       ea = __builtin_fmaf(e, v, ea);
     }
-  const float cs = exp2f((m - mn) * LOG2E);
+  const float cs = exp2_raw((m - mn) * LOG2E);
   s = __builtin_fmaf(s, cs, sum);
   a = __builtin_fmaf(a, cs, ea * invT);
   m = mn;
@@ -200,13 +215,14 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
 // scaled by 1/T and rounded to bf16, written straight from the accumulators (each lane
 // stores its four consecutive vocabulary rows of a token as 8 bytes; the lines of an
 // output row fill up in L2 across the wave's stores).
-__device__ __forceinline__ void grad_block(const Params& p, const floatx16 (&acc)[WV][WT], int t0, int vb, int wv,
+__device__ __forceinline__ void grad_block(const Params& p, const floatx4 (&acc)[WV][WT], int t0, int vb, int wv,
                                            int wt, int lane) {
-  const int r32 = lane & 31, half = lane >> 5;
+  const int r16 = lane & 15, quad = lane >> 4;
   const int cols = min(BV, p.V - vb * BV);
 #pragma unroll
   for (int j = 0; j < WT; ++j) {
-    const int n = t0 + wt * (WT * 32) + j * 32 + r32;
+    int n = t0 + wt * 32 + col_off(j) + r16;
+    asm volatile("" : "+v"(n));  // this token's addresses are formed here, not kept across the blocks
     if (n >= p.N) continue;
     const float lse = p.lse[n];
     const float glp = p.glp ? p.glp[n] : 0.0f;
@@ -217,39 +233,37 @@ __device__ __forceinline__ void grad_block(const Params& p, const floatx16 (&acc
     const float mb = lse * LOG2E, c1 = p.invT * LOG2E;
     uint16_t* row = p.out + (int64_t)n * p.os + (int64_t)vb * BV;
 #pragma unroll
-    for (int i = 0; i < WV; ++i)
+    for (int i = 0; i < WV; ++i) {
+      const int v0 = wv * 64 + row_off(i, 0) + 4 * quad;  // rows v0 .. v0+3
+      float gv[4];
 #pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const int v0 = wv * (WV * 32) + i * 32 + 8 * g4 + 4 * half;  // rows v0 .. v0+3
-        float gv[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float a = acc[i][j][4 * g4 + e];
-          const float z = a * p.invT;
-          const float pr = exp2f(__builtin_fmaf(a, c1, -mb));
-          const float onehot = (v0 + e == tl) ? 1.0f : 0.0f;
-          const float g = glp * (onehot - pr) + gent * pr * (cent - z);
-          gv[e] = g * p.invT;
-        }
-        uint2 w2;
-        w2.x = pack_bf16(gv[0], gv[1]);
-        w2.y = pack_bf16(gv[2], gv[3]);
-        if (v0 + 4 <= cols) {
-          *reinterpret_cast<uint2*>(row + v0) = w2;
-        } else {  // the vocabulary range ends inside these four rows
-          if (v0 < cols) row[v0] = (uint16_t)w2.x;
-          if (v0 + 1 < cols) row[v0 + 1] = (uint16_t)(w2.x >> 16);
-          if (v0 + 2 < cols) row[v0 + 2] = (uint16_t)w2.y;
-        }
+      for (int e = 0; e < 4; ++e) {
+        const float a = acc[i][j][e];
+        const float z = a * p.invT;
+        const float pr = exp2_raw(__builtin_fmaf(a, c1, -mb));
+        const float onehot = (v0 + e == tl) ? 1.0f : 0.0f;
+        const float g = glp * (onehot - pr) + gent * pr * (cent - z);
+        gv[e] = g * p.invT;
       }
+      uint2 w2;
+      w2.x = pack_bf16(gv[0], gv[1]);
+      w2.y = pack_bf16(gv[2], gv[3]);
+      if (v0 + 4 <= cols) {
+        *reinterpret_cast<uint2*>(row + v0) = w2;
+      } else {  // the vocabulary range ends inside these four rows
+        if (v0 < cols) row[v0] = (uint16_t)w2.x;
+        if (v0 + 1 < cols) row[v0 + 1] = (uint16_t)(w2.x >> 16);
+        if (v0 + 2 < cols) row[v0 + 2] = (uint16_t)w2.y;
+      }
+    }
   }
 }
 
 template <bool GRAD>
 __global__ __launch_bounds__(NT, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void fused_kernel(Params p) {
-  __shared__ __align__(16) unsigned char lds[LDS_BYTES];
+  __shared__ __align__(1024) unsigned char lds[LDS_BYTES];
 
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wv = wid % WAVES_V, wt = wid / WAVES_V;
   int tb, split;
   block_coords(p, blockIdx.x, tb, split);
@@ -267,165 +281,189 @@ __global__ __launch_bounds__(NT, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) v
     a_[j] = 0.0f;
   }
 
-  // Loader.  Wave w fills rows [R*w, R*w + R) of the weight block and of the token block,
-  // R = 256 / NWAVES; lane l of load q fills slot l%8 of row R*w + 8q + l/8 with global
-  // chunk (l%8) ^ swz(row) = (l%8) ^ swz(l/8) ^ 4*(q%2).  Chunks at or past the hidden
-  // size (only in a final partial stage) get bit 31 of the offset set, past every buffer,
-  // so they read zero.
-  constexpr int R = BV / NWAVES;
-  static_assert(BV == BT && R % 16 == 0 && ROWS_PER_LOAD == 8, "loader layout");
-  const int rows_x = min(BT, p.N - t0);
-  const __amdgpu_buffer_rsrc_t rx = rsrc(p.x + (int64_t)t0 * p.xs, (uint32_t)(rows_x * p.xs * 2));
-  const int lrow = wid * R + (lane >> 3);
-  const int lch = (lane & 7) ^ swz(lane >> 3);  // global chunk for even q; odd q load lch ^ 4
-  const uint32_t la = (uint32_t)(lrow * p.ws * 2), lb = (uint32_t)(lrow * p.xs * 2);
-  const uint32_t qa = (uint32_t)(8 * p.ws * 2), qb = (uint32_t)(8 * p.xs * 2);
-  int ld = 0, ld_k = 0, ld_vb = vb0;
+  // Loader.  A region is 128 rows of a stage; wave w fills its rows [16 w, 16 w + 16) by two
+  // loads, lane l of load q slot l%8 of row 16 w + 8 q + l/8 with global chunk
+  // (l%8) ^ swz(row) = (l%8) ^ swz(l/8) ^ 4 q.  Chunks at or past the hidden size (only in a
+  // final partial stage) and every chunk past the last stage get bit 31 of the offset set,
+  // past every buffer, so they read zero.
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)lds;
+  const v4i rx = rsrc(p.x + (int64_t)t0 * p.xs, (uint32_t)(min(BT, p.N - t0) * p.xs * 2));
+  const int lrow = wid * 16 + (lane >> 3);
+  uint32_t va[2], vx[2], past[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int ch = (lane & 7) ^ swz(lane >> 3) ^ (4 * q);
+    va[q] = (uint32_t)((lrow + 8 * q) * p.ws * 2) + 16 * ch;
+    vx[q] = (uint32_t)((lrow + 8 * q) * p.xs * 2) + 16 * ch;
+    past[q] = (uint32_t)((nst - 1) * BK + 8 * ch >= p.H) << 31;
+  }
+  const uint32_t half_w = (uint32_t)(BV / 2 * p.ws * 2), half_x = (uint32_t)(BT / 2 * p.xs * 2);
+  int ld = 0, ld_k = 0, ld_vb = vb0;  // the stage being loaded
   auto w_rsrc = [&](int vb) {
     const int v0 = vb * BV;
     return rsrc(p.w + (int64_t)v0 * p.ws, (uint32_t)(min(BV, p.V - v0) * p.ws * 2));
   };
-  __amdgpu_buffer_rsrc_t rw_ld = w_rsrc(vb0);
-  // The loads of one stage, one instruction per call q = 0 .. A_LOADS + B_LOADS - 1;
-  // advance() moves to the next stage afterwards.
-  uint32_t c0 = 0, c1 = 0;
-  unsigned char* ld_base = lds;
-  auto stage_setup = [&]() {
-    ld_base = lds + (ld & 1) * STAGE_BYTES;
-    const int k0 = ld_k * BK;
-    c0 = (uint32_t)((k0 + 8 * lch) * 2);
-    c1 = (uint32_t)((k0 + 8 * (lch ^ 4)) * 2);
-    if (k0 + BK > p.H) {
-      c0 |= (uint32_t)(k0 + 8 * lch >= p.H) << 31;
-      c1 |= (uint32_t)(k0 + 8 * (lch ^ 4) >= p.H) << 31;
-    }
-    if (ld >= total) {  // past the last stage: read nothing
-      c0 |= 1u << 31;
-      c1 |= 1u << 31;
-    }
+  v4i rw = w_rsrc(vb0);
+  auto load_region = [&](int reg) {
+    const bool is_w = reg < B0;
+    const uint32_t dst = lds0 + (uint32_t)((ld & 1) * STAGE_BYTES + reg * REGION_BYTES + wid * 16 * ROWB);
+    const uint32_t off = (uint32_t)(ld_k * ROWB) + (reg & 1) * (is_w ? half_w : half_x) + (ld >= total ? 1u << 31 : 0u);
+    const uint32_t tail = ld_k == nst - 1 ? ~0u : 0u;
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      load_lds(is_w ? rw : rx, ((is_w ? va[q] : vx[q]) + off) | (past[q] & tail), dst + q * 8 * ROWB);
   };
-  auto issue_one = [&](int q) {
-    if (q < A_LOADS)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw_ld, (lds_ptr_t)(ld_base + (wid * R + q * 8) * ROWB), 16,
-                                               la + q * qa + ((q & 1) ? c1 : c0), 0, 0, 0);
-    else
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr_t)(ld_base + (BV + wid * R + (q - A_LOADS) * 8) * ROWB),
-                                               16, lb + (q - A_LOADS) * qb + (((q - A_LOADS) & 1) ? c1 : c0), 0, 0, 0);
-  };
-  auto advance = [&]() {
+  auto next_load_stage = [&]() {
     ++ld;
     if (++ld_k == nst) {
       ld_k = 0;
-      if (++ld_vb < vb1) rw_ld = w_rsrc(ld_vb);
+      if (++ld_vb < vb1) rw = w_rsrc(ld_vb);
     }
   };
-  auto issue_next = [&]() {
-    stage_setup();
+
+  // Fragment reads: lane l takes row l%16 of each 16-row block and 8 values of chunk
+  // 4*ks + l/16, stored at slot chunk ^ swz(l%16).
+  const int r16 = lane & 15, quad = lane >> 4;
+  uint32_t ra[KS], rb[KS];
 #pragma unroll
-    for (int q = 0; q < A_LOADS + B_LOADS; ++q) issue_one(q);
-    advance();
+  for (int ks = 0; ks < KS; ++ks) {
+    const uint32_t c = (uint32_t)(r16 * ROWB + (((4 * ks + quad) ^ swz(r16)) << 4));
+    ra[ks] = (uint32_t)(wv * 64 * ROWB) + c;
+    rb[ks] = (uint32_t)(B0 * REGION_BYTES + wt * 32 * ROWB) + c;
+  }
+  floatx4 acc[WV][WT];
+  bf16x8 fa[4][KS], fb0[2][KS], fb1[2][KS];
+  auto frag = [&](uint32_t off) { return *reinterpret_cast<const bf16x8*>(lds + off); };
+  auto read_w = [&](int h) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) fa[i][ks] = frag(ra[ks] + h * REGION_BYTES + i * 16 * ROWB);
+  };
+  auto read_x = [&](bf16x8 (&fb)[2][KS], int ks, int h) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) fb[q][ks] = frag(rb[ks] + h * REGION_BYTES + q * 16 * ROWB);
+  };
+  // A quarter of the wave's tile over the stage: the vocabulary blocks of half h against the
+  // token blocks of half j; after(ks) runs behind k-step ks.
+  auto multiply = [&](auto first, int h, int j, const bf16x8 (&fb)[2][KS], auto&& after) {
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          floatx4& c = acc[4 * h + i][2 * j + q];
+          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i][ks], fb[q][ks], first && ks == 0 ? floatx4{} : c, 0, 0, 0);
+        }
+      after(ks);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_setprio(0);
+  };
+  auto nothing = [](int) {};
+
+  auto stage = [&](auto first) {
+    read_w(0);
+    load_region(B1);
+    wait_loads<LOADS_AHEAD>();
+    barrier();
+    multiply(first, 0, 0, fb0, nothing);
+    barrier();
+
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) read_x(fb1, ks, 1);
+    load_region(A1);
+    next_load_stage();
+    wait_loads<LOADS_AHEAD>();
+    barrier();
+    multiply(first, 0, 1, fb1, nothing);
+    barrier();
+
+    read_w(1);
+    load_region(B0);
+    wait_loads<LOADS_AHEAD>();
+    barrier();
+    multiply(first, 1, 1, fb1, nothing);
+    barrier();
+
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      ra[ks] ^= STAGE_BYTES;
+      rb[ks] ^= STAGE_BYTES;
+    }
+    load_region(A0);
+    wait_loads<LOADS_AHEAD>();
+    barrier();
+    multiply(first, 1, 0, fb0, [&](int ks) { read_x(fb0, ks, 0); });
   };
 
-  // Fragment reads: lane l takes row l%32 of each 32-row block and 8 values of chunk
-  // 2*ks + l/32, stored at slot chunk ^ swz(l%32).
-  const int r32 = lane & 31, half = lane >> 5;
-  const int fa_base = (wv * (WV * 32) + r32) * ROWB, fb_base = (BV + wt * (WT * 32) + r32) * ROWB;
-  int fch[KS];
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) fch[ks] = ((2 * ks + half) ^ swz(r32)) << 4;
-
-  // Prologue: stage 0 landed, its first fragments in registers, stage 1 on its way.
-  issue_next();
-  wait_loads();
+  // Prologue: all of stage 0 and the first half of stage 1 on their way, stage 0's first
+  // token fragments in registers, the second group one barrier behind.
+  load_region(B0);
+  load_region(A0);
+  load_region(B1);
+  load_region(A1);
+  next_load_stage();
+  load_region(B0);
+  load_region(A0);
+  wait_loads<LOADS_AHEAD>();
   barrier();
-  static_assert(KS == 4, "the stage body below is written for four k-steps");
-  static_assert(A_LOADS + B_LOADS <= WV * WT && WV + WT <= WV * WT, "interleave slots");
-  bf16x8 fa0[WV], fb0[WT], fa1[WV], fb1[WT];
-  read_frags(lds, fa_base + fch[0], fb_base + fch[0], fa0, fb0);
-  issue_next();
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) read_x(fb0, ks, 0);
+  if (wid >= NWAVES / 2) barrier();
 
-  // One barrier per stage.  Before it every wave has all of its reads of stage st back
-  // and its loads of stage st+1 landed, so after it stage st+1 is readable and the
-  // buffer of stage st takes the loads of stage st+2, a whole stage ahead of their use.
-  // Slot order: both token fragments first, then the weight fragments, so that each read
-  // is at least six multiplies ahead of its first use in the next k-step (multiplies run
-  // i-major: fb[0], fb[1] and fa[0] are needed first).
-  auto frag_read = [&](const unsigned char* stage, int c, bf16x8 (&fa)[WV], bf16x8 (&fb)[WT], int slot) {
-    if (slot < WT) fb[slot] = *reinterpret_cast<const bf16x8*>(stage + fb_base + c + slot * 32 * ROWB);
-    else if (slot < WV + WT) fa[slot - WT] = *reinterpret_cast<const bf16x8*>(stage + fa_base + c + (slot - WT) * 32 * ROWB);
-  };
-  int st = 0;  // index of the stage being multiplied in this workgroup's sequence
   for (int vb = vb0; vb < vb1; ++vb) {
-    floatx16 acc[WV][WT];
-#pragma unroll
-    for (int i = 0; i < WV; ++i)
-#pragma unroll
-      for (int j = 0; j < WT; ++j) acc[i][j] = floatx16{};
-    for (int kst = 0; kst < nst; ++kst, ++st) {
-      const unsigned char* stage = lds + (st & 1) * STAGE_BYTES;
-      mfma_set_x(acc, fa0, fb0, [&](int i) { frag_read(stage, fch[1], fa1, fb1, i); });
-      mfma_set_x(acc, fa1, fb1, [&](int i) { frag_read(stage, fch[2], fa0, fb0, i); });
-      mfma_set_x(acc, fa0, fb0, [&](int i) { frag_read(stage, fch[3], fa1, fb1, i); });
-      __builtin_amdgcn_s_waitcnt(0);  // own reads of stage st back, own loads of stage st+1 landed
+    stage(std::true_type{});
+    for (int kst = 1; kst < nst; ++kst) {
       barrier();
-      const unsigned char* next = lds + ((st + 1) & 1) * STAGE_BYTES;
-      // After the last stage the reads below fetch a buffer nobody uses and the loads
-      // read zeros (offsets past the buffer); both stay unconditional so the multiplies
-      // see one straight-line sequence.
-      stage_setup();
-      // Raised priority for the k-step that carries the next loads: the SIMD's two waves
-      // leave the barrier together, and the one that falls behind in this k-step wins
-      // the issue arbitration until it drops back, so both reach the next barrier
-      // together instead of one idling there (measured: 24.5 -> 22.9 ms at D).
-      __builtin_amdgcn_s_setprio(1);
-      mfma_set_x(acc, fa1, fb1, [&](int i) {
-        frag_read(next, fch[0], fa0, fb0, i);
-        if (i < A_LOADS + B_LOADS) issue_one(i);
-      });
-      __builtin_amdgcn_s_setprio(0);
-      advance();
+      stage(std::false_type{});
     }
-
-    // end of a vocabulary block: lane holds rows 8*(r/4) + 4*(lane/32) + r%4 of each
-    // 32-row block, at offsets from rbase that are compile-time constants
+    // end of a vocabulary block
     if constexpr (GRAD) {
       grad_block(p, acc, t0, vb, wv, wt, lane);
-      continue;
-    }
-    const int rbase = vb * BV + wv * (WV * 32) + 4 * half;
-    if ((vb + 1) * BV <= p.V) {
-#pragma unroll
-      for (int j = 0; j < WT; ++j) absorb<false>(acc, j, 0, p.invT, m_[j], s_[j], a_[j]);
     } else {
-      const int lim = p.V - rbase;
+      const int rbase = vb * BV + wv * 64 + 4 * quad;
+      if ((vb + 1) * BV <= p.V) {
 #pragma unroll
-      for (int j = 0; j < WT; ++j) absorb<true>(acc, j, lim, p.invT, m_[j], s_[j], a_[j]);
+        for (int j = 0; j < WT; ++j) absorb<false>(acc, j, 0, p.invT, m_[j], s_[j], a_[j]);
+      } else {
+        const int lim = p.V - rbase;
+#pragma unroll
+        for (int j = 0; j < WT; ++j) absorb<true>(acc, j, lim, p.invT, m_[j], s_[j], a_[j]);
+      }
     }
+    barrier();
   }
+  if (wid < NWAVES / 2) barrier();
+  wait_loads<0>();  // no load to LDS outlives the loop
 
   if constexpr (GRAD) return;
-  // combine the two lane halves (same tokens, interleaved rows), then the two vocab waves
+  // combine the lane quarters (same tokens, interleaved rows), then the two vocab waves
 #pragma unroll
-  for (int j = 0; j < WT; ++j) {
-    const float m2 = __shfl_xor(m_[j], 32), s2 = __shfl_xor(s_[j], 32), a2 = __shfl_xor(a_[j], 32);
-    merge(m_[j], s_[j], a_[j], m2, s2, a2);
-  }
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // no LDS loads in flight
+  for (int j = 0; j < WT; ++j)
+#pragma unroll
+    for (int o = 16; o <= 32; o <<= 1) {
+      const float m2 = __shfl_xor(m_[j], o), s2 = __shfl_xor(s_[j], o), a2 = __shfl_xor(a_[j], o);
+      merge(m_[j], s_[j], a_[j], m2, s2, a2);
+    }
   __syncthreads();
   static_assert(WAVES_V == 2, "the exchange below merges two vocabulary waves");
-  float4* xch = reinterpret_cast<float4*>(lds);  // [WAVES_T][WT*32] states of the waves with wv = 1
-  if (wv == 1 && lane < 32) {
+  float4* xch = reinterpret_cast<float4*>(lds);  // [BT] states of the waves with wv = 1
+  if (lane < 16) {
 #pragma unroll
-    for (int j = 0; j < WT; ++j) xch[wt * (WT * 32) + j * 32 + lane] = make_float4(m_[j], s_[j], a_[j], 0.0f);
+    for (int j = 0; j < WT; ++j)
+      if (wv == 1) xch[wt * 32 + col_off(j) + lane] = make_float4(m_[j], s_[j], a_[j], 0.0f);
   }
   __syncthreads();
-  if (wv == 0 && lane < 32) {
+  if (wv == 0 && lane < 16) {
 #pragma unroll
     for (int j = 0; j < WT; ++j) {
-      const float4 o = xch[wt * (WT * 32) + j * 32 + lane];
+      const int c = wt * 32 + col_off(j) + lane;
+      const float4 o = xch[c];
       merge(m_[j], s_[j], a_[j], o.x, o.y, o.z);
-      const int n = t0 + wt * (WT * 32) + j * 32 + lane;
-      if (n < p.N) p.part[(int64_t)split * p.N + n] = make_float4(m_[j], s_[j], a_[j], 0.0f);
+      if (t0 + c < p.N) p.part[(int64_t)split * p.N + t0 + c] = make_float4(m_[j], s_[j], a_[j], 0.0f);
     }
   }
 }
