@@ -56,22 +56,32 @@
 namespace dsv41 {
 namespace logprob {
 
-constexpr int WAVES_V = 2;                   // waves along the vocabulary
-constexpr int WAVES_T = 4;                   // waves along tokens
-constexpr int NWAVES = WAVES_V * WAVES_T;
-constexpr int NT = 64 * NWAVES;              // 8 waves, two per SIMD
+constexpr int NWAVES = 8;                    // two per SIMD
+constexpr int NT = 64 * NWAVES;
 constexpr int WV = 8;                        // 16-row MFMA blocks per wave along the vocabulary
 constexpr int WT = 4;                        // 16-column MFMA blocks per wave along tokens
-constexpr int BV = WAVES_V * WV * 16;        // 256 vocabulary rows per block
-constexpr int BT = WAVES_T * WT * 16;        // 256 tokens per workgroup
 constexpr int BK = 64;                       // hidden elements per stage
 constexpr int KS = BK / 32;                  // MFMA k-steps per stage
 constexpr int ROWB = BK * 2;                 // bytes per LDS row: one 128-byte cache line
-constexpr int STAGE_BYTES = (BV + BT) * ROWB;  // 64 KiB
-constexpr int LDS_BYTES = 2 * STAGE_BYTES;   // two stage buffers
-constexpr int A0 = 0, A1 = 1, B0 = 2, B1 = 3;  // a stage's regions: 128 weight or token rows each
-constexpr int REGION_BYTES = 128 * ROWB;
-constexpr int LOADS_AHEAD = 8;               // loads a wave keeps in flight past each wait
+// A workgroup's tile: WAVES_V waves along the vocabulary, the others along tokens.  The square
+// one (2: 256 x 256) loads least per multiply; the tall one (4: 512 rows x 128 tokens) pads
+// few tokens less, and fills all of a CU's LDS.
+template <int WAVES_V>
+struct Tile {
+  static constexpr int WAVES_T = NWAVES / WAVES_V;
+  static constexpr int BV = WAVES_V * WV * 16;  // vocabulary rows per block
+  static constexpr int BT = WAVES_T * WT * 16;  // tokens per workgroup
+  // a stage's regions, the halves of its weight rows and of its token rows, and their bytes
+  static constexpr int REGION_W = BV / 2 * ROWB, REGION_X = BT / 2 * ROWB;
+  static constexpr int STAGE = 2 * (REGION_W + REGION_X);
+  // loads of 8 rows per wave that fill a region, and loads a wave keeps in flight past each wait
+  static constexpr int LOADS_W = BV / 2 / 8 / NWAVES, LOADS_X = BT / 2 / 8 / NWAVES;
+  static constexpr int AHEAD = 2 * (LOADS_W + LOADS_X);
+};
+constexpr int A0 = 0, A1 = 1, B0 = 2, B1 = 3;  // the regions: weight halves, token halves
+constexpr int SQUARE = 2, TALL = 4;
+static_assert(2 * Tile<TALL>::STAGE <= 160 * 1024, "two stages fit the LDS");
+constexpr int MAX_PHASES = 2;
 constexpr int CU_COUNT = 256;                // MI355X
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float NEG_INF = -__builtin_huge_valf();
@@ -81,17 +91,26 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
+// A run of token blocks whose vocabulary is cut into the same number of ranges.
+struct Phase {
+  int first;   // its first workgroup (a multiple of 8)
+  int tb0, n_tb;
+  int splits;
+  int64_t part0;  // its states: part[part0 + split * tokens of the phase + token in the phase]
+};
+
 struct Params {
   const uint16_t* x;
   int64_t xs;
   const uint16_t* w;  // (backward: row vbeg of the head)
   int64_t ws;
   const int64_t* targets;
-  float4* part;  // [splits][N] (max z, sum e, sum e*z, unused)
+  float4* part;  // (max z, sum e, sum e*z, unused) of every range and token
   int N, H, V;   // (backward: V = rows of the vocabulary range)
   float invT;
-  int splits, n_vb, n_tb;
-  int group_t, group_s;  // XCD super-tile shape (0: linear mapping)
+  int gran;      // vocabulary ranges begin at multiples of gran rows
+  int n_ph;
+  Phase ph[MAX_PHASES];
   // backward only
   const float* lse;
   const float* ent;
@@ -101,6 +120,12 @@ struct Params {
   int64_t os;
   int vbeg;
 };
+
+// First row of range `split` of `splits`.
+__host__ __device__ inline int range_row(int V, int gran, int split, int splits) {
+  const int n = (V + gran - 1) / gran;
+  return min(V, (int)((int64_t)split * n / splits) * gran);
+}
 
 // Raw buffer descriptor: stride 0, reads at or past `bytes` return 0.
 __device__ __forceinline__ v4i rsrc(const void* base, uint32_t bytes) {
@@ -118,24 +143,27 @@ __device__ __forceinline__ void merge(float& m, float& s, float& a, float m2, fl
   m = mn;
 }
 
-// Block id -> (token block, vocabulary split).  Workgroups are dispatched round-robin
-// over the 8 XCDs; consecutive workgroups of one XCD form a group_t x group_s
-// rectangle of the (token block, split) grid, so they share operand panels in that
-// XCD's L2.  Falls back to split-fastest order when the grid does not tile.
-__device__ __forceinline__ void block_coords(const Params& p, int b, int& tb, int& split) {
-  const int total = p.n_tb * p.splits;
-  if (p.group_t > 0 && total % 8 == 0) {
-    const int xcd = b & 7, k = b >> 3;
-    const int gsz = p.group_t * p.group_s;
-    const int u = (k / gsz) * 8 + xcd;      // super tile index
-    const int in = k % gsz;
-    const int us_n = p.splits / p.group_s;  // super tiles along splits
-    tb = (u / us_n) * p.group_t + in / p.group_s;
-    split = (u % us_n) * p.group_s + in % p.group_s;
-  } else {
-    split = b % p.splits;
-    tb = b / p.splits;
+// Workgroup -> (phase, token block, vocabulary range); false: none (padding).  Workgroups are
+// dispatched round-robin over the 8 XCDs, and each XCD takes a run of consecutive items of the
+// phase, ordered so that the 32 it holds at a time form 8 token blocks x 4 ranges: they share
+// their operand panels in its L2.  (16 x 2 and 32 x 1 measured slower at 64 token blocks.)
+__device__ __forceinline__ bool item_of(const Params& p, int b, int& tb, int& split, int& phase) {
+  phase = p.n_ph > 1 && b >= p.ph[1].first ? 1 : 0;
+  const int n_tb = phase ? p.ph[1].n_tb : p.ph[0].n_tb, splits = phase ? p.ph[1].splits : p.ph[0].splits;
+  const int items = n_tb * splits, per_xcd = (items + 7) / 8;
+  const int l = b - (phase ? p.ph[1].first : 0);
+  const int idx = (l & 7) * per_xcd + (l >> 3);
+  if ((l >> 3) >= per_xcd || idx >= items) return false;
+  const int group = idx / (8 * splits), in = idx - group * 8 * splits;
+  const int wide = min(8, n_tb - 8 * group);
+  int t = in % wide;
+  split = in / wide;
+  if (wide == 8 && splits % 4 == 0) {  // the same 8 x 4, ranges fastest (0.4% faster at 8 x 32)
+    t = in % 32 / 4;
+    split = in / 32 * 4 + in % 4;
   }
+  tb = (phase ? p.ph[1].tb0 : p.ph[0].tb0) + 8 * group + t;
+  return true;
 }
 
 // Bank-group swizzle of the 16-byte chunks of LDS row `row`.  It depends only on
@@ -171,20 +199,22 @@ __device__ __forceinline__ float exp2_raw(float x) { return __builtin_amdgcn_exp
 // Vocabulary row of block i, accumulator register r, and token column of block j, relative to
 // the lane's first ones: a wave holds rows [64 wv, +64) and tokens [32 wt, +32) of both halves
 // of the workgroup's tile, a lane rows 4 (lane / 16) + r of each block and token lane % 16.
-constexpr int row_off(int i, int r) { return (i / 4) * (BV / 2) + (i % 4) * 16 + r; }
-constexpr int col_off(int j) { return (j / 2) * (BT / 2) + (j % 2) * 16; }
+template <class TL>
+constexpr int row_off(int i, int r) { return (i / 4) * (TL::BV / 2) + (i % 4) * 16 + r; }
+template <class TL>
+constexpr int col_off(int j) { return (j / 2) * (TL::BT / 2) + (j % 2) * 16; }
 
 // Folds one vocabulary block into the running (max z, sum e, sum e*z) of token column j.
 // Rows at offsets >= lim lie past the vocabulary (their weights read as zero) and are
 // skipped when MASK is set.
-template <bool MASK>
+template <class TL, bool MASK>
 __device__ __forceinline__ void absorb(const floatx4 (&acc)[WV][WT], int j, int lim, float invT, float& m,
                                        float& s, float& a) {
   float mx = NEG_INF;
 #pragma unroll
   for (int i = 0; i < WV; ++i)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) mx = fmaxf(mx, (!MASK || row_off(i, r) < lim) ? acc[i][j][r] : NEG_INF);
+    for (int r = 0; r < 4; ++r) mx = fmaxf(mx, (!MASK || row_off<TL>(i, r) < lim) ? acc[i][j][r] : NEG_INF);
   const float mn = fmaxf(m, mx * invT);  // invT > 0: the max commutes with the scaling
   if (mn == NEG_INF) return;
   const float c1 = invT * LOG2E, mb = mn * LOG2E;
@@ -194,7 +224,7 @@ __device__ __forceinline__ void absorb(const floatx4 (&acc)[WV][WT], int j, int 
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const float v = acc[i][j][r];
-      const float e = exp2_raw((!MASK || row_off(i, r) < lim) ? __builtin_fmaf(v, c1, -mb) : NEG_INF);
+      const float e = exp2_raw((!MASK || row_off<TL>(i, r) < lim) ? __builtin_fmaf(v, c1, -mb) : NEG_INF);
       sum += e;
       ea = __builtin_fmaf(e, v, ea);
     }
@@ -215,26 +245,27 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
 // scaled by 1/T and rounded to bf16, written straight from the accumulators (each lane
 // stores its four consecutive vocabulary rows of a token as 8 bytes; the lines of an
 // output row fill up in L2 across the wave's stores).
-__device__ __forceinline__ void grad_block(const Params& p, const floatx4 (&acc)[WV][WT], int t0, int vb, int wv,
-                                           int wt, int lane) {
+template <class TL>
+__device__ __forceinline__ void grad_block(const Params& p, const floatx4 (&acc)[WV][WT], int t0, int vr, int vend,
+                                           int wv, int wt, int lane) {
   const int r16 = lane & 15, quad = lane >> 4;
-  const int cols = min(BV, p.V - vb * BV);
+  const int cols = vend - vr;  // (a whole block or less)
 #pragma unroll
   for (int j = 0; j < WT; ++j) {
-    int n = t0 + wt * 32 + col_off(j) + r16;
+    int n = t0 + wt * 32 + col_off<TL>(j) + r16;
     asm volatile("" : "+v"(n));  // this token's addresses are formed here, not kept across the blocks
     if (n >= p.N) continue;
     const float lse = p.lse[n];
     const float glp = p.glp ? p.glp[n] : 0.0f;
     const float gent = p.gent ? p.gent[n] : 0.0f;
     const float cent = p.gent ? lse - p.ent[n] : 0.0f;  // lse - entropy = E[z]
-    const int64_t tt = p.targets[n] - p.vbeg - (int64_t)vb * BV;
-    const int tl = (tt >= 0 && tt < BV) ? (int)tt : -1;  // target row within this block, if there
+    const int64_t tt = p.targets[n] - p.vbeg - vr;
+    const int tl = (tt >= 0 && tt < TL::BV) ? (int)tt : -1;  // target row within this block, if there
     const float mb = lse * LOG2E, c1 = p.invT * LOG2E;
-    uint16_t* row = p.out + (int64_t)n * p.os + (int64_t)vb * BV;
+    uint16_t* row = p.out + (int64_t)n * p.os + vr;
 #pragma unroll
     for (int i = 0; i < WV; ++i) {
-      const int v0 = wv * 64 + row_off(i, 0) + 4 * quad;  // rows v0 .. v0+3
+      const int v0 = wv * 64 + row_off<TL>(i, 0) + 4 * quad;  // rows v0 .. v0+3
       float gv[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -259,19 +290,23 @@ __device__ __forceinline__ void grad_block(const Params& p, const floatx4 (&acc)
   }
 }
 
-template <bool GRAD>
+template <bool GRAD, int WAVES_V>
 __global__ __launch_bounds__(NT, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void fused_kernel(Params p) {
-  __shared__ __align__(1024) unsigned char lds[LDS_BYTES];
+  using TL = Tile<WAVES_V>;
+  constexpr int BV = TL::BV, BT = TL::BT;
+  __shared__ __align__(1024) unsigned char lds[2 * TL::STAGE];
 
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wv = wid % WAVES_V, wt = wid / WAVES_V;
-  int tb, split;
-  block_coords(p, blockIdx.x, tb, split);
+  int tb, split, phase;
+  if (!item_of(p, blockIdx.x, tb, split, phase)) return;
   const int t0 = tb * BT;
-  const int vb0 = (int)((int64_t)split * p.n_vb / p.splits);
-  const int vb1 = (int)((int64_t)(split + 1) * p.n_vb / p.splits);
-  const int nst = (p.H + BK - 1) / BK;  // stages per vocabulary block
-  const int total = (vb1 - vb0) * nst;  // stages of this workgroup
+  const int splits = phase ? p.ph[1].splits : p.ph[0].splits;
+  const int v0 = range_row(p.V, p.gran, split, splits), v1 = range_row(p.V, p.gran, split + 1, splits);
+  const int nst = (p.H + BK - 1) / BK;                // stages per vocabulary block
+  const int nblk = (v1 - v0 + BV - 1) / BV;           // its vocabulary blocks, of `step` rows each
+  const int step = p.gran < BV ? ((v1 - v0 + nblk - 1) / nblk + 15) / 16 * 16 : BV;
+  const int total = nblk * nst;                       // stages of this workgroup
 
   float m_[WT], s_[WT], a_[WT];
 #pragma unroll
@@ -281,43 +316,49 @@ __global__ __launch_bounds__(NT, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) v
     a_[j] = 0.0f;
   }
 
-  // Loader.  A region is 128 rows of a stage; wave w fills its rows [16 w, 16 w + 16) by two
-  // loads, lane l of load q slot l%8 of row 16 w + 8 q + l/8 with global chunk
-  // (l%8) ^ swz(row) = (l%8) ^ swz(l/8) ^ 4 q.  Chunks at or past the hidden size (only in a
+  // Loader.  Wave w fills an eighth of a region's rows by loads of 8 rows, lane l slot l%8 of
+  // row l/8 with global chunk (l%8) ^ swz(row).  Chunks at or past the hidden size (only in a
   // final partial stage) and every chunk past the last stage get bit 31 of the offset set,
   // past every buffer, so they read zero.
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)lds;
   const v4i rx = rsrc(p.x + (int64_t)t0 * p.xs, (uint32_t)(min(BT, p.N - t0) * p.xs * 2));
-  const int lrow = wid * 16 + (lane >> 3);
-  uint32_t va[2], vx[2], past[2];
+  uint32_t va[2], past_w[2], vx[2], past_x[2];  // of even and odd loads
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
-    const int ch = (lane & 7) ^ swz(lane >> 3) ^ (4 * q);
-    va[q] = (uint32_t)((lrow + 8 * q) * p.ws * 2) + 16 * ch;
-    vx[q] = (uint32_t)((lrow + 8 * q) * p.xs * 2) + 16 * ch;
-    past[q] = (uint32_t)((nst - 1) * BK + 8 * ch >= p.H) << 31;
+    const int rw = wid * 8 * TL::LOADS_W + 8 * q + (lane >> 3), rt = wid * 8 * TL::LOADS_X + 8 * q + (lane >> 3);
+    const int cw = (lane & 7) ^ swz(rw), ct = (lane & 7) ^ swz(rt);
+    va[q] = (uint32_t)(rw * p.ws * 2) + 16 * cw;
+    vx[q] = (uint32_t)(rt * p.xs * 2) + 16 * ct;
+    past_w[q] = (uint32_t)((nst - 1) * BK + 8 * cw >= p.H) << 31;
+    past_x[q] = (uint32_t)((nst - 1) * BK + 8 * ct >= p.H) << 31;
   }
   const uint32_t half_w = (uint32_t)(BV / 2 * p.ws * 2), half_x = (uint32_t)(BT / 2 * p.xs * 2);
-  int ld = 0, ld_k = 0, ld_vb = vb0;  // the stage being loaded
-  auto w_rsrc = [&](int vb) {
-    const int v0 = vb * BV;
-    return rsrc(p.w + (int64_t)v0 * p.ws, (uint32_t)(min(BV, p.V - v0) * p.ws * 2));
+  const uint32_t rows16 = (uint32_t)(16 * p.ws * 2);
+  int ld = 0, ld_k = 0, ld_v = v0;  // the stage being loaded
+  auto w_rsrc = [&](int v) {
+    return rsrc(p.w + (int64_t)v * p.ws, (uint32_t)(min(step, v1 - v) * p.ws * 2));
   };
-  v4i rw = w_rsrc(vb0);
+  v4i rw = w_rsrc(v0);
   auto load_region = [&](int reg) {
     const bool is_w = reg < B0;
-    const uint32_t dst = lds0 + (uint32_t)((ld & 1) * STAGE_BYTES + reg * REGION_BYTES + wid * 16 * ROWB);
+    const uint32_t at = (uint32_t)((ld & 1) * TL::STAGE) +
+                        (uint32_t)(is_w ? (reg & 1) * TL::REGION_W : 2 * TL::REGION_W + (reg & 1) * TL::REGION_X);
+    const uint32_t dst = lds0 + at + (uint32_t)(wid * (is_w ? TL::LOADS_W : TL::LOADS_X) * 8 * ROWB);
     const uint32_t off = (uint32_t)(ld_k * ROWB) + (reg & 1) * (is_w ? half_w : half_x) + (ld >= total ? 1u << 31 : 0u);
     const uint32_t tail = ld_k == nst - 1 ? ~0u : 0u;
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
-      load_lds(is_w ? rw : rx, ((is_w ? va[q] : vx[q]) + off) | (past[q] & tail), dst + q * 8 * ROWB);
+    for (int q = 0; q < (is_w ? TL::LOADS_W : TL::LOADS_X); ++q)
+      load_lds(is_w ? rw : rx,
+               is_w ? (va[q & 1] + (off + (uint32_t)(q / 2) * rows16)) | (past_w[q & 1] & tail)
+                    : (vx[q & 1] + off) | (past_x[q & 1] & tail),
+               dst + q * 8 * ROWB);
   };
   auto next_load_stage = [&]() {
     ++ld;
     if (++ld_k == nst) {
       ld_k = 0;
-      if (++ld_vb < vb1) rw = w_rsrc(ld_vb);
+      ld_v += step;
+      if (ld_v < v1) rw = w_rsrc(ld_v);
     }
   };
 
@@ -329,8 +370,9 @@ __global__ __launch_bounds__(NT, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) v
   for (int ks = 0; ks < KS; ++ks) {
     const uint32_t c = (uint32_t)(r16 * ROWB + (((4 * ks + quad) ^ swz(r16)) << 4));
     ra[ks] = (uint32_t)(wv * 64 * ROWB) + c;
-    rb[ks] = (uint32_t)(B0 * REGION_BYTES + wt * 32 * ROWB) + c;
+    rb[ks] = (uint32_t)(2 * TL::REGION_W + wt * 32 * ROWB) + c;
   }
+  uint32_t flip = TL::STAGE;  // to the other stage buffer
   floatx4 acc[WV][WT];
   bf16x8 fa[4][KS], fb0[2][KS], fb1[2][KS];
   auto frag = [&](uint32_t off) { return *reinterpret_cast<const bf16x8*>(lds + off); };
@@ -338,11 +380,11 @@ __global__ __launch_bounds__(NT, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) v
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) fa[i][ks] = frag(ra[ks] + h * REGION_BYTES + i * 16 * ROWB);
+      for (int i = 0; i < 4; ++i) fa[i][ks] = frag(ra[ks] + h * TL::REGION_W + i * 16 * ROWB);
   };
   auto read_x = [&](bf16x8 (&fb)[2][KS], int ks, int h) {
 #pragma unroll
-    for (int q = 0; q < 2; ++q) fb[q][ks] = frag(rb[ks] + h * REGION_BYTES + q * 16 * ROWB);
+    for (int q = 0; q < 2; ++q) fb[q][ks] = frag(rb[ks] + h * TL::REGION_X + q * 16 * ROWB);
   };
   // A quarter of the wave's tile over the stage: the vocabulary blocks of half h against the
   // token blocks of half j; after(ks) runs behind k-step ks.
@@ -367,7 +409,7 @@ __global__ __launch_bounds__(NT, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) v
   auto stage = [&](auto first) {
     read_w(0);
     load_region(B1);
-    wait_loads<LOADS_AHEAD>();
+    wait_loads<TL::AHEAD>();
     barrier();
     multiply(first, 0, 0, fb0, nothing);
     barrier();
@@ -376,25 +418,27 @@ __global__ __launch_bounds__(NT, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) v
     for (int ks = 0; ks < KS; ++ks) read_x(fb1, ks, 1);
     load_region(A1);
     next_load_stage();
-    wait_loads<LOADS_AHEAD>();
+    wait_loads<TL::AHEAD>();
     barrier();
     multiply(first, 0, 1, fb1, nothing);
     barrier();
 
     read_w(1);
     load_region(B0);
-    wait_loads<LOADS_AHEAD>();
+    wait_loads<TL::AHEAD>();
     barrier();
     multiply(first, 1, 1, fb1, nothing);
     barrier();
 
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      ra[ks] ^= STAGE_BYTES;
-      rb[ks] ^= STAGE_BYTES;
+      ra[ks] = TL::STAGE == 1 << 16 ? ra[ks] ^ TL::STAGE : ra[ks] + flip;
+      rb[ks] = TL::STAGE == 1 << 16 ? rb[ks] ^ TL::STAGE : rb[ks] + flip;
+      asm volatile("" : "+v"(ra[ks]), "+v"(rb[ks]));  // here, not among the multiplies (1.5%)
     }
+    flip = 0u - flip;
     load_region(A0);
-    wait_loads<LOADS_AHEAD>();
+    wait_loads<TL::AHEAD>();
     barrier();
     multiply(first, 1, 0, fb0, [&](int ks) { read_x(fb0, ks, 0); });
   };
@@ -408,13 +452,13 @@ __global__ __launch_bounds__(NT, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) v
   next_load_stage();
   load_region(B0);
   load_region(A0);
-  wait_loads<LOADS_AHEAD>();
+  wait_loads<TL::AHEAD>();
   barrier();
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) read_x(fb0, ks, 0);
   if (wid >= NWAVES / 2) barrier();
 
-  for (int vb = vb0; vb < vb1; ++vb) {
+  for (int v = v0; v < v1; v += step) {
     stage(std::true_type{});
     for (int kst = 1; kst < nst; ++kst) {
       barrier();
@@ -422,17 +466,14 @@ __global__ __launch_bounds__(NT, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) v
     }
     // end of a vocabulary block
     if constexpr (GRAD) {
-      grad_block(p, acc, t0, vb, wv, wt, lane);
+      grad_block<TL>(p, acc, t0, v, min(v1, v + step), wv, wt, lane);
+    } else if (step == BV && v + BV <= v1) {
+#pragma unroll
+      for (int j = 0; j < WT; ++j) absorb<TL, false>(acc, j, 0, p.invT, m_[j], s_[j], a_[j]);
     } else {
-      const int rbase = vb * BV + wv * 64 + 4 * quad;
-      if ((vb + 1) * BV <= p.V) {
+      const int lim = min(v1, v + step) - (v + wv * 64 + 4 * quad);
 #pragma unroll
-        for (int j = 0; j < WT; ++j) absorb<false>(acc, j, 0, p.invT, m_[j], s_[j], a_[j]);
-      } else {
-        const int lim = p.V - rbase;
-#pragma unroll
-        for (int j = 0; j < WT; ++j) absorb<true>(acc, j, lim, p.invT, m_[j], s_[j], a_[j]);
-      }
+      for (int j = 0; j < WT; ++j) absorb<TL, true>(acc, j, lim, p.invT, m_[j], s_[j], a_[j]);
     }
     barrier();
   }
@@ -449,33 +490,41 @@ __global__ __launch_bounds__(NT, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) v
       merge(m_[j], s_[j], a_[j], m2, s2, a2);
     }
   __syncthreads();
-  static_assert(WAVES_V == 2, "the exchange below merges two vocabulary waves");
-  float4* xch = reinterpret_cast<float4*>(lds);  // [BT] states of the waves with wv = 1
-  if (lane < 16) {
+  float4* xch = reinterpret_cast<float4*>(lds);  // [WAVES_V - 1][BT] states of the waves with wv > 0
+  if (wv > 0 && lane < 16) {
 #pragma unroll
     for (int j = 0; j < WT; ++j)
-      if (wv == 1) xch[wt * 32 + col_off(j) + lane] = make_float4(m_[j], s_[j], a_[j], 0.0f);
+      xch[(wv - 1) * BT + wt * 32 + col_off<TL>(j) + lane] = make_float4(m_[j], s_[j], a_[j], 0.0f);
   }
   __syncthreads();
   if (wv == 0 && lane < 16) {
+    const int tok0 = (phase ? p.ph[1].tb0 : p.ph[0].tb0) * BT;  // the phase's first token, and its tokens
+    const int ntok = min(p.N - tok0, (phase ? p.ph[1].n_tb : p.ph[0].n_tb) * BT);
+    float4* out = p.part + (phase ? p.ph[1].part0 : p.ph[0].part0) + (int64_t)split * ntok - tok0;
 #pragma unroll
     for (int j = 0; j < WT; ++j) {
-      const int c = wt * 32 + col_off(j) + lane;
-      const float4 o = xch[c];
-      merge(m_[j], s_[j], a_[j], o.x, o.y, o.z);
-      if (t0 + c < p.N) p.part[(int64_t)split * p.N + t0 + c] = make_float4(m_[j], s_[j], a_[j], 0.0f);
+      const int c = wt * 32 + col_off<TL>(j) + lane;
+#pragma unroll
+      for (int u = 0; u < WAVES_V - 1; ++u) {
+        const float4 o = xch[u * BT + c];
+        merge(m_[j], s_[j], a_[j], o.x, o.y, o.z);
+      }
+      if (t0 + c < p.N) out[t0 + c] = make_float4(m_[j], s_[j], a_[j], 0.0f);
     }
   }
 }
 
 struct MergeParams {
-  const float4* part;  // [splits][N] split states, or [shards][N] shard states (combine)
+  const float4* part;  // the ranges' states (see Phase), or [shards][N] shard states (combine)
   const uint16_t* x;
   int64_t xs;
   const uint16_t* w;
   int64_t ws;
   const int64_t* targets;
-  int N, H, V, splits;
+  int N, H, V, shards;
+  int BT;              // tokens per block of the phases
+  int n_ph;
+  Phase ph[MAX_PHASES];
   int64_t voff;  // shard: global id of w's first row
   float invT;
   const float* behavior;
@@ -526,8 +575,17 @@ __global__ __launch_bounds__(256) void merge_kernel(MergeParams q) {
     }
   }
   float m = NEG_INF, s = 0.0f, a = 0.0f, zs = NEG_INF;
-  for (int k = lane; k < q.splits; k += 64) {
-    const float4 o = q.part[(int64_t)k * q.N + n];
+  // the token's states: a column of its phase's, or of the shards'
+  int parts = q.shards, step = q.N;
+  const float4* col = q.part + n;
+  if (MODE != MERGE_COMBINE) {
+    const Phase ph = q.n_ph > 1 && n >= q.ph[1].tb0 * q.BT ? q.ph[1] : q.ph[0];
+    parts = ph.splits;
+    step = min(q.N - ph.tb0 * q.BT, ph.n_tb * q.BT);
+    col = q.part + ph.part0 + (n - ph.tb0 * q.BT);
+  }
+  for (int k = lane; k < parts; k += 64) {
+    const float4 o = col[(int64_t)k * step];
     merge(m, s, a, o.x, o.y, o.z);
     if (MODE == MERGE_COMBINE) zs = fmaxf(zs, o.w);
   }
@@ -564,29 +622,107 @@ __global__ __launch_bounds__(256) void merge_kernel(MergeParams q) {
 }
 
 struct Plan {
-  int splits, n_vb, n_tb, group_t, group_s;
+  bool tall;
+  int gran, n_ph, grid;
+  Phase ph[MAX_PHASES];
   size_t workspace;
 };
 
-// One workgroup per CU: split the vocabulary so token blocks x splits fills the machine,
-// at least one vocabulary block per split (ranges are spread evenly).
-int split_count(int n_tb, int n_vb) {
-  const int want = n_tb > 0 ? std::max(1, CU_COUNT / n_tb) : 1;
-  return std::max(1, std::min(want, n_vb));
+// Microseconds: one stage of the square and of the tall tile, a block's softmax epilogue, the
+// start of a workgroup until its first operands have landed, and a megabyte of weights from HBM
+// (measured: 2048 and 600 tokens of 7168 -> 129280, 8192 of 2048 -> 151936, one token).
+constexpr double STAGE_US = 1.36, TALL_STAGE_US = 1.55, BLOCK_US = 3.0, FILL_US = 3.0, WEIGHT_US = 1.0 / 5.9;
+
+// The best cut of n_tb token blocks, all of whose workgroups sweep one range of n_vb vocabulary
+// blocks of block_us each: ranges that fill the CUs one to four times, by the longest CU's time.
+struct Cut {
+  int splits;
+  double us;
+};
+Cut cut(int n_tb, int n_vb, double block_us, double weights_us) {
+  Cut best{1, 1e300};
+  for (int k = 1; k <= 4; ++k) {
+    const int s = std::max(1, std::min((int)((int64_t)CU_COUNT * k / n_tb), n_vb));
+    const double rounds = (double)(((int64_t)n_tb * s + CU_COUNT - 1) / CU_COUNT);
+    const double us = rounds * ((n_vb + s - 1) / s * block_us + FILL_US);
+    // (a tenth of the multiplies shows beside a stream of weights that takes longer)
+    const double all = std::max(us, weights_us) + 0.1 * us;
+    if (all < best.us * 0.995) best = Cut{s, all};
+  }
+  return best;
 }
 
-// XCD super tiles of 32 workgroups (token blocks x splits) when the grid tiles.
-void xcd_groups(Plan* pl) {
-  pl->group_t = 0;
-  pl->group_s = 0;
-  for (int gs : {4, 8, 2, 16, 1, 32}) {
-    const int gt = 32 / gs;
-    if (pl->splits % gs == 0 && pl->n_tb % gt == 0 && (pl->n_tb * pl->splits) % (8 * 32) == 0) {
-      pl->group_t = gt;
-      pl->group_s = gs;
-      break;
+// Tile, phases and ranges of N tokens over V rows of hidden size H.
+//
+// The vocabulary is cut so that token blocks x ranges fill the CUs; where no count of ranges
+// does (65 token blocks: three ranges leave 61 CUs idle), a power of two of the token blocks
+// fills them exactly and the others, finely cut, follow in the same launch.  The tall tile's
+// half as many tokens take the place of the square's where padding 256-token blocks costs more
+// (331 tokens: three blocks of 128 against two of 256).  Each phase streams the weights once,
+// shared by its token blocks in L2, so one of few tokens costs at least that stream; ranges
+// then begin at any multiple of 16 rows, so that every CU streams the same share.
+// Measured before and after, each pair on one box (7168 -> 129280 unless noted): 64 tokens of
+// 2048 -> 151936 168 -> 159 us, 128 tokens 357 -> 335, 331 tokens 627 -> 571, 600 tokens
+// 980 -> 891, 10000 tokens 13.63 -> 12.77 ms, 16640 tokens 24.35 -> 22.16 ms.  The choice is
+// within 3% of the best of both tiles and of one to four ranges per CU at 22 counts of tokens.
+void plan_items(int N, int H, int V, int64_t ws, Plan* pl) {
+  *pl = Plan{};
+  if (N == 0) return;
+  const int nst = (H + BK - 1) / BK;
+  const double weights_us = 2e-6 * V * H * WEIGHT_US;
+  double best = 1e300;
+  for (const bool tall : {false, true}) {
+    if (tall && Tile<TALL>::BV * ws * 2 >= (1ll << 31)) continue;  // 32-bit offsets within a block
+    const int BT = tall ? Tile<TALL>::BT : Tile<SQUARE>::BT, BV = tall ? Tile<TALL>::BV : Tile<SQUARE>::BV;
+    const int n_tb = (N + BT - 1) / BT, n_vb = (V + BV - 1) / BV;
+    const double block_us = nst * (tall ? TALL_STAGE_US : STAGE_US) + BLOCK_US;
+    const Cut one = cut(n_tb, n_vb, block_us, weights_us);
+    if (one.us < best) {
+      best = one.us;
+      pl->tall = tall;
+      pl->n_ph = 1;
+      pl->ph[0] = Phase{0, 0, n_tb, one.splits, 0};
+    }
+    int p2 = 1;
+    while (2 * p2 < n_tb && p2 < CU_COUNT) p2 *= 2;
+    const int n1 = n_tb > CU_COUNT ? n_tb / CU_COUNT * CU_COUNT : p2;
+    if (n1 < n_tb && n_tb > 2) {
+      const Cut a = cut(n1, n_vb, block_us, weights_us), b = cut(n_tb - n1, n_vb, block_us, weights_us);
+      if (a.us + b.us < best) {
+        best = a.us + b.us;
+        pl->tall = tall;
+        pl->n_ph = 2;
+        pl->ph[0] = Phase{0, 0, n1, a.splits, 0};
+        pl->ph[1] = Phase{0, n1, n_tb - n1, b.splits, 0};
+      }
     }
   }
+  const int BT = pl->tall ? Tile<TALL>::BT : Tile<SQUARE>::BT;
+  pl->gran = pl->tall ? Tile<TALL>::BV : Tile<SQUARE>::BV;
+  if (pl->n_ph == 1 && pl->ph[0].n_tb * pl->ph[0].splits <= CU_COUNT && best < 1.5 * weights_us) {
+    pl->gran = 16;
+    pl->ph[0].splits = std::max(1, std::min(CU_COUNT / pl->ph[0].n_tb, (V + 15) / 16));
+  }
+  int64_t states = 0;
+  int first = 0;
+  for (int i = 0; i < pl->n_ph; ++i) {
+    Phase& ph = pl->ph[i];
+    ph.first = first;
+    first += (ph.n_tb * ph.splits + 7) / 8 * 8;
+    ph.part0 = states;
+    states += (int64_t)ph.splits * std::min(N - ph.tb0 * BT, ph.n_tb * BT);
+  }
+  pl->grid = first;
+  pl->workspace = (size_t)states * sizeof(float4);
+}
+
+template <bool GRAD>
+void launch(const Plan& pl, Params& p, hipStream_t s) {
+  p.gran = pl.gran;
+  p.n_ph = pl.n_ph;
+  for (int i = 0; i < MAX_PHASES; ++i) p.ph[i] = pl.ph[i];
+  if (pl.tall) hipLaunchKernelGGL((fused_kernel<GRAD, TALL>), dim3(pl.grid), dim3(NT), 0, s, p);
+  else hipLaunchKernelGGL((fused_kernel<GRAD, SQUARE>), dim3(pl.grid), dim3(NT), 0, s, p);
 }
 
 int plan(const dsv41_logprob_desc* d, Plan* pl) {
@@ -600,7 +736,7 @@ int plan(const dsv41_logprob_desc* d, Plan* pl) {
     return fail(DSV41_E_INVALID, "row strides must be >= hidden and multiples of 8 elements");
   if (((uintptr_t)d->x | (uintptr_t)d->w) % 16)
     return fail(DSV41_E_INVALID, "hidden states and head weight must be 16-byte aligned");
-  if ((int64_t)BV * d->w_row_stride * 2 >= (1ll << 31) || (int64_t)BT * d->x_row_stride * 2 >= (1ll << 31))
+  if (256 * std::max(d->w_row_stride, d->x_row_stride) * 2 >= (1ll << 31))
     return fail(DSV41_E_UNSUPPORTED, "row stride too large for 32-bit block offsets");
   if (!(isfinite(d->temperature) && d->temperature > 0.0f))
     return fail(DSV41_E_INVALID, "temperature must be finite and positive");
@@ -609,11 +745,7 @@ int plan(const dsv41_logprob_desc* d, Plan* pl) {
     return fail(DSV41_E_INVALID, "is_cap must be finite and positive");
   if (d->n_tokens > 0 && (!d->x || !d->w || !d->targets || !d->out_logprob))
     return fail(DSV41_E_INVALID, "x, w, targets and out_logprob are required");
-  pl->n_vb = (d->vocab + BV - 1) / BV;
-  pl->n_tb = (d->n_tokens + BT - 1) / BT;
-  pl->splits = split_count(pl->n_tb, pl->n_vb);
-  xcd_groups(pl);
-  pl->workspace = (size_t)pl->splits * (size_t)d->n_tokens * sizeof(float4);
+  plan_items(d->n_tokens, d->hidden, d->vocab, d->w_row_stride, pl);
   return DSV41_OK;
 }
 
@@ -630,7 +762,7 @@ int plan_grad(const dsv41_logprob_grad_desc* d, Plan* pl) {
     return fail(DSV41_E_INVALID, "row strides must be >= hidden and multiples of 8 elements");
   if (((uintptr_t)d->x | (uintptr_t)d->w | (uintptr_t)d->out) % 16)
     return fail(DSV41_E_INVALID, "hidden states, head weight and output must be 16-byte aligned");
-  if ((int64_t)BV * d->w_row_stride * 2 >= (1ll << 31) || (int64_t)BT * d->x_row_stride * 2 >= (1ll << 31))
+  if (256 * std::max(d->w_row_stride, d->x_row_stride) * 2 >= (1ll << 31))
     return fail(DSV41_E_UNSUPPORTED, "row stride too large for 32-bit block offsets");
   if (!(isfinite(d->temperature) && d->temperature > 0.0f))
     return fail(DSV41_E_INVALID, "temperature must be finite and positive");
@@ -641,10 +773,7 @@ int plan_grad(const dsv41_logprob_grad_desc* d, Plan* pl) {
   if (d->n_tokens > 0 && (!d->x || !d->w || !d->targets || !d->lse || !d->out))
     return fail(DSV41_E_INVALID, "x, w, targets, lse and out are required");
   if (d->grad_entropy && !d->entropy) return fail(DSV41_E_INVALID, "an entropy gradient requires the entropies");
-  pl->n_vb = (d->vocab_end - d->vocab_begin + BV - 1) / BV;
-  pl->n_tb = (d->n_tokens + BT - 1) / BT;
-  pl->splits = split_count(pl->n_tb, pl->n_vb);
-  xcd_groups(pl);
+  plan_items(d->n_tokens, d->hidden, d->vocab_end - d->vocab_begin, d->w_row_stride, pl);
   pl->workspace = 0;
   return DSV41_OK;
 }
@@ -670,11 +799,6 @@ extern "C" int dsv41_logprob_grad_run(const dsv41_logprob_grad_desc* d, void* st
   p.H = d->hidden;
   p.V = d->vocab_end - d->vocab_begin;
   p.invT = 1.0f / d->temperature;
-  p.splits = pl.splits;
-  p.n_vb = pl.n_vb;
-  p.n_tb = pl.n_tb;
-  p.group_t = pl.group_t;
-  p.group_s = pl.group_s;
   p.lse = d->lse;
   p.ent = d->entropy;
   p.glp = d->grad_logprob;
@@ -682,7 +806,7 @@ extern "C" int dsv41_logprob_grad_run(const dsv41_logprob_grad_desc* d, void* st
   p.out = static_cast<uint16_t*>(d->out);
   p.os = d->out_row_stride;
   p.vbeg = d->vocab_begin;
-  hipLaunchKernelGGL(fused_kernel<true>, dim3(pl.n_tb * pl.splits), dim3(NT), 0, static_cast<hipStream_t>(stream), p);
+  launch<true>(pl, p, static_cast<hipStream_t>(stream));
   DSV41_HIP_CHECK(hipGetLastError());
   return DSV41_OK;
 }
@@ -713,12 +837,7 @@ extern "C" int dsv41_logprob_run(const dsv41_logprob_desc* d, void* workspace, s
   p.H = d->hidden;
   p.V = d->vocab;
   p.invT = 1.0f / d->temperature;
-  p.splits = pl.splits;
-  p.n_vb = pl.n_vb;
-  p.n_tb = pl.n_tb;
-  p.group_t = pl.group_t;
-  p.group_s = pl.group_s;
-  hipLaunchKernelGGL(fused_kernel<false>, dim3(pl.n_tb * pl.splits), dim3(NT), 0, s, p);
+  launch<false>(pl, p, s);
   DSV41_HIP_CHECK(hipGetLastError());
   MergeParams q{};
   q.part = p.part;
@@ -730,7 +849,9 @@ extern "C" int dsv41_logprob_run(const dsv41_logprob_desc* d, void* workspace, s
   q.N = d->n_tokens;
   q.H = d->hidden;
   q.V = d->vocab;
-  q.splits = pl.splits;
+  q.BT = pl.tall ? Tile<TALL>::BT : Tile<SQUARE>::BT;
+  q.n_ph = pl.n_ph;
+  for (int i = 0; i < MAX_PHASES; ++i) q.ph[i] = pl.ph[i];
   q.invT = p.invT;
   q.behavior = d->behavior;
   q.is_cap = d->is_cap;
@@ -800,12 +921,7 @@ extern "C" int dsv41_logprob_shard_run(const dsv41_logprob_shard_desc* d, void* 
   p.H = d->hidden;
   p.V = d->vocab;
   p.invT = 1.0f / d->temperature;
-  p.splits = pl.splits;
-  p.n_vb = pl.n_vb;
-  p.n_tb = pl.n_tb;
-  p.group_t = pl.group_t;
-  p.group_s = pl.group_s;
-  hipLaunchKernelGGL(fused_kernel<false>, dim3(pl.n_tb * pl.splits), dim3(NT), 0, s, p);
+  launch<false>(pl, p, s);
   DSV41_HIP_CHECK(hipGetLastError());
   MergeParams q{};
   q.part = p.part;
@@ -817,7 +933,9 @@ extern "C" int dsv41_logprob_shard_run(const dsv41_logprob_shard_desc* d, void* 
   q.N = d->n_tokens;
   q.H = d->hidden;
   q.V = d->vocab;
-  q.splits = pl.splits;
+  q.BT = pl.tall ? Tile<TALL>::BT : Tile<SQUARE>::BT;
+  q.n_ph = pl.n_ph;
+  for (int i = 0; i < MAX_PHASES; ++i) q.ph[i] = pl.ph[i];
   q.voff = d->vocab_offset;
   q.invT = p.invT;
   q.state_out = reinterpret_cast<float4*>(d->out_state);
@@ -841,7 +959,7 @@ extern "C" int dsv41_logprob_combine_run(const dsv41_logprob_combine_desc* d, vo
   MergeParams q{};
   q.part = reinterpret_cast<const float4*>(d->states);
   q.N = d->n_tokens;
-  q.splits = d->n_shards;
+  q.shards = d->n_shards;
   q.behavior = d->behavior;
   q.is_cap = d->is_cap;
   q.lp = d->out_logprob;
