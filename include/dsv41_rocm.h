@@ -4,7 +4,8 @@
  *
  * Plain C: pointers, sizes and PODs only. Every device pointer is a HIP device
  * address owned by the caller; the library never allocates or frees device
- * memory, never synchronises the stream, and launches only on `stream`.
+ * memory, never synchronises the stream (dsv41_check_wait alone does), and launches only on
+ * `stream`.
  *
  * Return codes: 0 on success, a negative DSV41_E_* code before any launch on a
  * bad argument. dsv41_last_error() then holds a thread-local message whose text
@@ -551,6 +552,14 @@ int dsv41_token_tis_run(const dsv41_token_tis_desc* desc, void* workspace, size_
 size_t dsv41_grpo_workspace_bytes(const dsv41_grpo_desc* desc);
 int dsv41_grpo_run(const dsv41_grpo_desc* desc, void* workspace, size_t workspace_bytes,
                    void* stream /* hipStream_t */);
+
+/* What a checked call asks after its launches: returns 1 when some of the n statuses is
+ * nonzero, plus 2 when some of the n_ids ids lies outside [0, limit) (0: neither), or a negative
+ * error.  Unlike every other entry point it waits for the stream.  `flags` is one int32 of pinned
+ * host memory that nothing else uses during the call.  Serves the checks of rollout.py:145-146
+ * and model.py:725-727. */
+int dsv41_check_wait(const int32_t* status, int64_t n, const int64_t* ids, int64_t n_ids, int64_t limit,
+                     int32_t* flags, void* stream /* hipStream_t */);
 
 #ifdef __cplusplus
 }

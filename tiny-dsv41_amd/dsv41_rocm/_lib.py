@@ -312,6 +312,7 @@ EXPORTS = (
     "dsv41_sampler_full_mass_run",
     "dsv41_sampler_full_draw_run",
     "dsv41_sampler_full_finish_run",
+    "dsv41_check_wait",
 )
 
 _lock = threading.Lock()
@@ -371,6 +372,9 @@ def _bind(lib: ctypes.CDLL) -> ctypes.CDLL:
         getattr(lib, name).argtypes = [ctypes.POINTER(SamplerFullShardDesc), ctypes.c_void_p]
     lib.dsv41_sampler_full_finish_run.restype = ctypes.c_int
     lib.dsv41_sampler_full_finish_run.argtypes = [ctypes.POINTER(SamplerFullFinishDesc), ctypes.c_void_p]
+    lib.dsv41_check_wait.restype = ctypes.c_int
+    lib.dsv41_check_wait.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64,
+                                    ctypes.c_void_p, ctypes.c_void_p]
     return lib
 
 

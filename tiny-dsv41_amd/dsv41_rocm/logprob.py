@@ -29,6 +29,7 @@ from typing import Optional
 import torch
 
 from . import _lib
+from ._check import any_set
 
 
 def _status_error(status: torch.Tensor) -> None:
@@ -41,7 +42,9 @@ def _status_error(status: torch.Tensor) -> None:
         raise ValueError("raw rollout importance weights underflowed")
 
 
-def _prepare(hidden, weight, targets, temperature):
+def _prepare(hidden, weight, targets, temperature, check_targets=True):
+    """Arguments in kernel form.  Without check_targets the caller checks the target ids itself
+    (the kernels give NaN for one outside the vocabulary)."""
     if not math.isfinite(temperature) or temperature <= 0:
         raise ValueError("temperature must be finite and positive")
     if hidden.ndim != 2 or weight.ndim != 2 or hidden.shape[1] != weight.shape[1]:
@@ -53,7 +56,8 @@ def _prepare(hidden, weight, targets, temperature):
     targets = targets.to(device=hidden.device, dtype=torch.int64).reshape(-1)
     if targets.numel() != n:
         raise ValueError("one target is required per token")
-    if n and bool(((targets < 0) | (targets >= v)).any()):
+    targets = targets.contiguous()
+    if check_targets and any_set(None, targets, v)[1]:
         raise ValueError("target token ID is outside the model vocabulary")
     if h % 8:
         raise ValueError("hidden size must be a multiple of 8")
@@ -63,7 +67,7 @@ def _prepare(hidden, weight, targets, temperature):
         hidden = hidden.contiguous()
     if weight.stride(1) != 1 or weight.stride(0) % 8 or weight.data_ptr() % 16:
         weight = weight.contiguous()
-    return hidden, weight, targets.contiguous()
+    return hidden, weight, targets
 
 
 def _forward(hidden, weight, targets, temperature, behavior, is_cap):
@@ -226,14 +230,19 @@ def selected_log_probs(
     in ``hidden`` and ``weight`` (log-prob and entropy), like the reference expression under
     autograd.
     """
-    hidden, weight, targets = _prepare(hidden, weight, targets, temperature)
+    # with check, the ids are checked beside the statuses: one synchronisation for both
+    hidden, weight, targets = _prepare(hidden, weight, targets, temperature, check_targets=not check)
     if torch.is_grad_enabled() and (hidden.requires_grad or weight.requires_grad):
         lp, ent, ratio, status = _SelectedLogProbs.apply(hidden, weight, targets, temperature, behavior, is_cap)
         ratio = ratio if behavior is not None else None
     else:
         lp, ent, ratio, _, status = _forward(hidden, weight, targets, temperature, behavior, is_cap)
-    if check and hidden.shape[0] and bool((status != 0).any()):
-        _status_error(status)
+    if check:
+        bad_status, bad_target = any_set(status, targets, weight.shape[0])
+        if bad_target:
+            raise ValueError("target token ID is outside the model vocabulary")
+        if bad_status:
+            _status_error(status)
     return lp, ent, ratio
 
 
@@ -306,7 +315,7 @@ def combine_states(states: torch.Tensor, *, behavior: Optional[torch.Tensor] = N
     with torch.cuda.device(dev):
         rc = lib.dsv41_logprob_combine_run(ctypes.byref(d), torch.cuda.current_stream(dev).cuda_stream)
     _lib.check(rc)
-    if check and n and bool((status != 0).any()):
+    if check and any_set(status)[0]:
         _status_error(status)
     return lp, ent, ratio
 
@@ -322,8 +331,16 @@ def token_log_probs(hidden: torch.Tensor, weight: torch.Tensor, targets: torch.T
     """Drop-in for model.py:679-684 (``_token_log_probs``): fp32 [B, T] with the selected
     targets' log-probs where ``mask`` is set and zeros elsewhere."""
     mask = mask.to(torch.bool)
-    selected = hidden[mask]
+    if mask.shape != targets.shape or mask.shape != hidden.shape[:-1] or mask.device != hidden.device:
+        selected = hidden[mask]  # (shapes that only partly match, or raise as indexing does)
+        if selected.shape[0] == 0:
+            return torch.zeros(mask.shape, dtype=torch.float32, device=hidden.device)
+        lp = selected_log_probs(selected, weight, targets[mask], temperature)[0]
+        return lp.new_zeros(mask.shape).masked_scatter(mask, lp)
+    # the mask's places once (one wait for their count), for both gathers and the scatter
+    at = mask.nonzero(as_tuple=True)
+    selected = hidden[at]
     if selected.shape[0] == 0:
         return torch.zeros(mask.shape, dtype=torch.float32, device=hidden.device)
-    lp = selected_log_probs(selected, weight, targets[mask], temperature)[0]
-    return lp.new_zeros(mask.shape).masked_scatter(mask, lp)
+    lp = selected_log_probs(selected, weight, targets[at], temperature)[0]
+    return lp.new_zeros(mask.shape).index_put(at, lp)

@@ -26,6 +26,7 @@ from typing import Optional
 import torch
 
 from . import _lib
+from ._check import any_set
 
 
 @dataclass
@@ -216,7 +217,7 @@ def sample(
         rc = lib.dsv41_sampler_run(_lib.ctypes.byref(desc), _device_ptr(workspace), ws_bytes, stream)
     _lib.check(rc)
     if check:
-        if bool((status != 0).any()):
+        if any_set(status)[0]:
             _status_error(status)
     return SampleResult(ids, lps, kept, status)
 
@@ -415,7 +416,7 @@ def merge_shards(
         rc = lib.dsv41_sampler_merge_run(_lib.ctypes.byref(d), stream)
     _lib.check(rc)
     if check:
-        if bool((out_status != 0).any()):
+        if any_set(out_status)[0]:
             _status_error(out_status)
     return SampleResult(ids, lps, kept, out_status)
 
@@ -649,7 +650,7 @@ def full_shard_finish(
         rc = lib.dsv41_sampler_full_finish_run(_lib.ctypes.byref(d), stream)
     _lib.check(rc)
     if check:
-        if bool((status != 0).any()):
+        if any_set(status)[0]:
             _status_error(status)
     return SampleResult(ids, lps, kept, status)
 
@@ -696,6 +697,6 @@ def replay_log_probs(
         rc = lib.dsv41_sampler_run(_lib.ctypes.byref(desc), None, 0, stream)
     _lib.check(rc)
     if check:
-        if bool((status != 0).any()):
+        if any_set(status)[0]:
             _status_error(status)
     return lps

@@ -27,6 +27,7 @@ import ctypes
 import math
 from typing import Sequence
 
+import numpy as np
 import torch
 
 from . import _lib
@@ -60,13 +61,46 @@ _CHECKS = (
 )
 
 
+def _vector(value, like):
+    """A detached float32 vector on like's device."""
+    if type(value) is torch.Tensor and value.dtype == torch.float32 and value.device == like.device:
+        return value.detach() if value.requires_grad else value
+    return torch.as_tensor(value, dtype=torch.float32, device=like.device).detach()
+
+
+def _upload(lengths, advantages, device):
+    """The responses' offsets (int64 [R + 1]) and advantages (float32 [R]) on the device, in one
+    copy where the advantages are on the host."""
+    offsets = np.zeros(len(lengths) + 1, dtype=np.int64)
+    np.cumsum(lengths, out=offsets[1:])
+    if advantages.device.type != "cpu":
+        return torch.from_numpy(offsets).to(device), advantages.to(device).contiguous()
+    cut = offsets.nbytes
+    host = torch.empty(cut + 4 * len(lengths), dtype=torch.uint8, pin_memory=True)
+    view = host.numpy()
+    view[:cut] = offsets.view(np.uint8)
+    view[cut:] = advantages.contiguous().numpy().view(np.uint8)
+    both = host.to(device, non_blocking=True)  # (torch keeps the pinned block until the copy is over)
+    return both[:cut].view(torch.int64), both[cut:].view(torch.float32)
+
+
+def _report(n_metrics, R, device):
+    """Metrics (float64) and statuses (int32 [R]) in one block, so that they come back in one copy."""
+    block = torch.empty(8 * n_metrics + 4 * R, dtype=torch.uint8, device=device)
+    return block, block.data_ptr(), block.data_ptr() + 8 * n_metrics
+
+
+def _read_report(block, n_metrics):
+    host = block.cpu().numpy()
+    return host[:8 * n_metrics].view(np.float64).tolist(), host[8 * n_metrics:].view(np.int32)
+
+
 def _run(current, old, behavior, advantages, offsets, clip_eps, is_cap, want_grad):
     R = advantages.numel()
     dev = current.device
-    loss = torch.empty(1, dtype=torch.float32, device=dev)
+    loss = torch.empty((), dtype=torch.float32, device=dev)
     grad = torch.empty_like(current) if want_grad else None
-    metrics = torch.empty(len(METRIC_KEYS), dtype=torch.float64, device=dev)
-    status = torch.empty(R, dtype=torch.int32, device=dev)
+    report, metrics, status = _report(len(METRIC_KEYS), R, dev)
     d = _lib.TokenTisDesc()
     d.struct_size = ctypes.sizeof(_lib.TokenTisDesc)
     d.n_responses, d.n_tokens = R, current.numel()
@@ -74,7 +108,7 @@ def _run(current, old, behavior, advantages, offsets, clip_eps, is_cap, want_gra
     d.current, d.native_old, d.behavior = current.data_ptr(), old.data_ptr(), behavior.data_ptr()
     d.advantages = advantages.data_ptr()
     d.clip_eps, d.is_cap = clip_eps, is_cap
-    d.out_loss, d.out_metrics, d.out_status = loss.data_ptr(), metrics.data_ptr(), status.data_ptr()
+    d.out_loss, d.out_metrics, d.out_status = loss.data_ptr(), metrics, status
     d.out_grad = grad.data_ptr() if grad is not None else None
     lib = _lib.load()
     ws_bytes = lib.dsv41_token_tis_workspace_bytes(ctypes.byref(d))
@@ -82,19 +116,19 @@ def _run(current, old, behavior, advantages, offsets, clip_eps, is_cap, want_gra
     with torch.cuda.device(dev):
         rc = lib.dsv41_token_tis_run(ctypes.byref(d), ws.data_ptr(), ws_bytes, torch.cuda.current_stream(dev).cuda_stream)
     _lib.check(rc)
-    return loss[0], grad, metrics, status
+    return loss, grad, report
 
 
 class _TokenTIS(torch.autograd.Function):
     @staticmethod
     def forward(ctx, current, old, behavior, advantages, offsets, clip_eps, is_cap):
-        loss, grad, metrics, status = _run(current, old, behavior, advantages, offsets, clip_eps, is_cap, True)
+        loss, grad, report = _run(current, old, behavior, advantages, offsets, clip_eps, is_cap, True)
         ctx.save_for_backward(grad)
-        ctx.mark_non_differentiable(metrics, status)
-        return loss, metrics, status
+        ctx.mark_non_differentiable(report)
+        return loss, report
 
     @staticmethod
-    def backward(ctx, g_loss, g_metrics, g_status):
+    def backward(ctx, g_loss, g_report):
         (grad,) = ctx.saved_tensors
         return grad * g_loss, None, None, None, None, None, None
 
@@ -126,8 +160,8 @@ def decoupled_token_tis_loss(
         if not isinstance(current, torch.Tensor) or current.ndim != 1 or current.numel() == 0:
             raise ValueError("each policy log-probability tensor must be a nonempty vector")
         current = current.float()
-        old = torch.as_tensor(native_old_log_probs[index], dtype=torch.float32, device=current.device).detach()
-        behavior = torch.as_tensor(behavior_log_probs[index], dtype=torch.float32, device=current.device).detach()
+        old = _vector(native_old_log_probs[index], current)
+        behavior = _vector(behavior_log_probs[index], current)
         if old.shape != current.shape or behavior.shape != current.shape:
             raise ValueError("native-old, behavior and policy response lengths must match")
         currents.append(current)
@@ -137,20 +171,16 @@ def decoupled_token_tis_loss(
     dev = currents[0].device
     if dev.type != "cuda":
         raise ValueError("log probabilities must be on the GPU (libdsv41hip has no CPU path)")
-    offsets = torch.zeros(size + 1, dtype=torch.int64)
-    offsets[1:] = torch.cumsum(torch.tensor(lengths, dtype=torch.int64), 0)
+    offsets, adv = _upload(lengths, advantage_values, dev)
     cur = torch.cat(currents)
     old = torch.cat(olds).contiguous()
     beh = torch.cat(behaviors).contiguous()
-    adv = advantage_values.to(dev).contiguous()
-    offsets = offsets.to(dev)
     if torch.is_grad_enabled() and cur.requires_grad:
-        loss, metrics, status = _TokenTIS.apply(cur.contiguous(), old, beh, adv, offsets, clip_eps, is_cap)
+        loss, report = _TokenTIS.apply(cur.contiguous(), old, beh, adv, offsets, clip_eps, is_cap)
     else:
-        loss, _, metrics, status = _run(cur.detach().contiguous(), old, beh, adv, offsets, clip_eps, is_cap, False)
-    host = torch.cat([metrics, status.double()]).cpu()  # the one host copy
-    values, st = host[:len(METRIC_KEYS)].tolist(), [int(v) for v in host[len(METRIC_KEYS):].tolist()]
-    for bits in st:
+        loss, _, report = _run(cur.detach().contiguous(), old, beh, adv, offsets, clip_eps, is_cap, False)
+    values, st = _read_report(report, len(METRIC_KEYS))  # the one host copy
+    for bits in st[st != 0].tolist():
         if bits:
             for bit, message in _CHECKS:
                 if bits & bit:
@@ -183,10 +213,9 @@ _GRPO_CHECKS = (
 def _run_grpo(current, behavior, reference, advantages, offsets, clip_eps, kl_beta, want_grad):
     R = advantages.numel()
     dev = current.device
-    loss = torch.empty(1, dtype=torch.float32, device=dev)
+    loss = torch.empty((), dtype=torch.float32, device=dev)
     grad = torch.empty_like(current) if want_grad else None
-    metrics = torch.empty(len(GRPO_METRIC_KEYS), dtype=torch.float64, device=dev)
-    status = torch.empty(R, dtype=torch.int32, device=dev)
+    report, metrics, status = _report(len(GRPO_METRIC_KEYS), R, dev)
     d = _lib.GrpoDesc()
     d.struct_size = ctypes.sizeof(_lib.GrpoDesc)
     d.n_responses, d.n_tokens = R, current.numel()
@@ -195,7 +224,7 @@ def _run_grpo(current, behavior, reference, advantages, offsets, clip_eps, kl_be
     d.reference = reference.data_ptr() if reference is not None else None
     d.advantages = advantages.data_ptr()
     d.clip_eps, d.kl_beta = clip_eps, kl_beta
-    d.out_loss, d.out_metrics, d.out_status = loss.data_ptr(), metrics.data_ptr(), status.data_ptr()
+    d.out_loss, d.out_metrics, d.out_status = loss.data_ptr(), metrics, status
     d.out_grad = grad.data_ptr() if grad is not None else None
     lib = _lib.load()
     ws_bytes = lib.dsv41_grpo_workspace_bytes(ctypes.byref(d))
@@ -203,20 +232,19 @@ def _run_grpo(current, behavior, reference, advantages, offsets, clip_eps, kl_be
     with torch.cuda.device(dev):
         rc = lib.dsv41_grpo_run(ctypes.byref(d), ws.data_ptr(), ws_bytes, torch.cuda.current_stream(dev).cuda_stream)
     _lib.check(rc)
-    return loss[0], grad, metrics, status
+    return loss, grad, report
 
 
 class _Grpo(torch.autograd.Function):
     @staticmethod
     def forward(ctx, current, behavior, reference, advantages, offsets, clip_eps, kl_beta):
-        loss, grad, metrics, status = _run_grpo(current, behavior, reference, advantages, offsets, clip_eps,
-                                                kl_beta, True)
+        loss, grad, report = _run_grpo(current, behavior, reference, advantages, offsets, clip_eps, kl_beta, True)
         ctx.save_for_backward(grad)
-        ctx.mark_non_differentiable(metrics, status)
-        return loss, metrics, status
+        ctx.mark_non_differentiable(report)
+        return loss, report
 
     @staticmethod
-    def backward(ctx, g_loss, g_metrics, g_status):
+    def backward(ctx, g_loss, g_report):
         (grad,) = ctx.saved_tensors
         return grad * g_loss, None, None, None, None, None, None
 
@@ -252,7 +280,7 @@ def grpo_loss(
         if current.ndim != 1 or current.numel() == 0:
             raise ValueError("each policy log-probability tensor must be a nonempty vector")
         current = current.float()
-        behavior = torch.as_tensor(behavior_log_probs[index], dtype=torch.float32, device=current.device).detach()
+        behavior = _vector(behavior_log_probs[index], current)
         if behavior.shape != current.shape:
             raise ValueError("behavior and policy response lengths must match")
         if kl_beta:
@@ -266,21 +294,16 @@ def grpo_loss(
     dev = currents[0].device
     if dev.type != "cuda":
         raise ValueError("log probabilities must be on the GPU (libdsv41hip has no CPU path)")
-    offsets = torch.zeros(size + 1, dtype=torch.int64)
-    offsets[1:] = torch.cumsum(torch.tensor(lengths, dtype=torch.int64), 0)
+    offsets, adv = _upload(lengths, advantage_values, dev)
     cur = torch.cat(currents)
     beh = torch.cat(behaviors).contiguous()
     ref = torch.cat(references).contiguous() if kl_beta else None
-    adv = advantage_values.to(dev).contiguous()
-    offsets = offsets.to(dev)
     if torch.is_grad_enabled() and cur.requires_grad:
-        loss, metrics, status = _Grpo.apply(cur.contiguous(), beh, ref, adv, offsets, clip_eps, kl_beta)
+        loss, report = _Grpo.apply(cur.contiguous(), beh, ref, adv, offsets, clip_eps, kl_beta)
     else:
-        loss, _, metrics, status = _run_grpo(cur.detach().contiguous(), beh, ref, adv, offsets, clip_eps, kl_beta,
-                                             False)
-    host = torch.cat([metrics, status.double()]).cpu()
-    values, st = host[:len(GRPO_METRIC_KEYS)].tolist(), [int(v) for v in host[len(GRPO_METRIC_KEYS):].tolist()]
-    for bits in st:
+        loss, _, report = _run_grpo(cur.detach().contiguous(), beh, ref, adv, offsets, clip_eps, kl_beta, False)
+    values, st = _read_report(report, len(GRPO_METRIC_KEYS))
+    for bits in st[st != 0].tolist():
         if bits:
             for bit, message in _GRPO_CHECKS:
                 if bits & bit:
