@@ -493,7 +493,9 @@ const char* dsv41_last_error(void);
  * 2048-aligned vocabulary slices of at least 6144 ids (up to about 256 workgroups in
  * all, S*top_k <= 4096) that
  * each leave their local top_k keys, a count and a status for a merge kernel on the
- * same stream; none otherwise. */
+ * same stream; for a full-vocabulary batch that is spread over the GPU (at most 128 rows, and
+ * bf16 ones of 257 to 448), rows*(12*ceil(vocab/256)+4*S) and alignment, which replays and the
+ * larger batches may do without (they then run one workgroup per row); none otherwise. */
 size_t dsv41_sampler_workspace_bytes(const dsv41_sampler_desc* desc);
 int dsv41_sampler_run(const dsv41_sampler_desc* desc, void* workspace, size_t workspace_bytes,
                       void* stream /* hipStream_t */);

@@ -1,5 +1,6 @@
-"""Vector loads over rows that end inside a vector: ids, kept sets and statuses exactly the
-oracle's, log-probs within 1e-4, whatever lies behind the rows."""
+"""Small top-p and min-p batches cut into slices (small_*_kernel), full-vocabulary batches spread
+over the GPU beyond 128 rows, and vector loads over rows that end inside a vector: ids, kept sets
+and statuses exactly the oracle's, log-probs within 1e-4, at the edges of their ranges."""
 
 import numpy as np
 import pytest
@@ -40,6 +41,64 @@ def _agrees(full, vocab, u, hist, **knobs):
     assert np.array_equal(got.kept.cpu().numpy(), kept)
     fine = status == 0
     assert np.max(np.abs(got.logprobs.cpu().numpy()[fine] - lps[fine]), initial=0.0) <= 1e-4
+
+
+PENALTIES = [(0, {}), (40, {"repetition_penalty": 1.2}), (300, {"presence_penalty": 0.4, "frequency_penalty": 0.3}),
+             (77, {"repetition_penalty": 0.7, "presence_penalty": -0.5})]
+
+
+@pytest.mark.parametrize("rows,vocab", [(1, 18433), (3, 20011), (17, 24577), (128, 18500), (129, 18500), (2, 151851)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("history,pen", PENALTIES)
+def test_top_p_slices(rows, vocab, dtype, history, pen):
+    for i, top_p in enumerate((0.9, 0.01, 0.9995)):
+        full, u, hist = _batch(rows, vocab, dtype, 7 * rows + i, history)
+        _agrees(full, vocab, u, hist, temperature=(0.8, 1.0, 0.6)[i], top_p=top_p, **pen)
+    _agrees(full, vocab, u, hist, temperature=0.8, top_p=0.9, greedy=True, **pen)
+
+
+@pytest.mark.parametrize("rows,vocab", [(1, 18433), (3, 20011), (200, 18500), (256, 18500), (257, 18500), (2, 151851)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("history,pen", PENALTIES)
+def test_min_p_slices(rows, vocab, dtype, history, pen):
+    for i, knobs in enumerate(({"min_p": 0.05}, {"min_p": 0.3, "top_p": 0.8}, {"min_p": 0.001})):
+        full, u, hist = _batch(rows, vocab, dtype, 11 * rows + i, history)
+        _agrees(full, vocab, u, hist, temperature=(0.8, 1.0, 0.6)[i], **knobs, **pen)
+    _agrees(full, vocab, u, hist, temperature=0.8, min_p=0.05, greedy=True, **pen)
+
+
+@pytest.mark.parametrize("knobs", [{"top_p": 0.9}, {"min_p": 0.05}])
+def test_slices_of_odd_rows(knobs):
+    """Flat rows (more tokens at the boundary than the lists hold: the fallback), one far token, a
+    NaN, an infinity, the type's lowest value, a bad uniform and a bad history id."""
+    V = 20011
+    full, u, hist = _batch(9, V, torch.float32, 5, 30)
+    full[0, :V] = 0.25
+    full[1, :V] = -50.0
+    full[1, 15000] = 50.0
+    full[2, 19999] = float("nan")
+    full[3, 3] = float("inf")
+    full[4, 77] = float("-inf")
+    full[5, :V:3] = torch.finfo(torch.float32).min
+    u[6] = 1.5
+    hist[7, 5] = V
+    full[8, :V] = torch.round(full[8, :V])  # many ties
+    _agrees(full, V, u, hist, temperature=1.0, repetition_penalty=1.1, **knobs)
+    _agrees(full, V, u, None, temperature=0.7, **knobs)
+
+
+@pytest.mark.parametrize("rows", [128, 129, 256, 257, 300, 448, 449])
+@pytest.mark.parametrize("history,pen", PENALTIES[:3])
+def test_spread_full_vocabulary(rows, history, pen):
+    import dsv41_rocm
+
+    V = 9001
+    full, u, hist = _batch(rows, V, torch.bfloat16, rows, history)
+    _agrees(full, V, u, hist, temperature=0.7, **pen)
+    logits, h = full.to(DEV)[:, :V], None if hist is None else hist.to(DEV)
+    r = dsv41_rocm.sample(logits, uniforms=u.to(DEV), history=h, temperature=0.7, **pen)
+    again = dsv41_rocm.replay_log_probs(logits, r.ids, history=h, temperature=0.7, **pen)
+    assert torch.equal(again, r.logprobs)  # bit for bit, whichever way either was cut
 
 
 @pytest.mark.parametrize("vocab", [255, 1001, 4095, 4098, 9003, 151851])

@@ -68,6 +68,13 @@ constexpr int TOPP_NT = 1024;
 constexpr int TOPP_BINS = 4096;                // 32 octaves of (max - z) x 128 steps
 constexpr int TOPP_BIN_BASE = 100 << 7;        // octave 0 is [2^-27, 2^-26); smaller -> bin 0
 constexpr int TOPP_CAP = 4096;                 // list / boundary-bin tokens topp_kernel holds
+// Small top-p / min-p batches (small_*_kernel): at most so many rows (one workgroup per row is as
+// fast at 200 of top-p, 144 us both, and at 400 of min-p, 113 us), cut into so many slices in all
+// (top-p, whose bins cost every slice the same: 48 rows 74 us at 768, 79 at 1536, 87 at 3072).
+constexpr int SMALL_TOPP_ROWS = 128, SMALL_MINP_ROWS = 256;
+constexpr int SMALL_TOPP_GRID = 768, SMALL_MINP_GRID = 1536;
+constexpr int SMALL_MIN_W = 2048;
+constexpr size_t SMALL_MAX_LDS = 64 * 1024;
 static_assert(TOPP_CAP <= TOPP_BINS, "the boundary bin's tokens from the list go to the bins' space");
 constexpr size_t LDS_LIMIT = 160 * 1024;
 // Cache policy of the row streams: nt (non-temporal).  A pass reads each logit and history
@@ -102,8 +109,14 @@ constexpr int DRAW_ARGMAX = 8;      // first largest logit without its log-prob:
 // Exact masses of the inverse-CDF draws are formed per chunk of MASS_CHUNK consecutive ids
 // of the row (or slice), against the chunk's own maximum.
 constexpr int MASS_CHUNK = 256;
-// FULL batches of at most this many rows are spread over the GPU
+// FULL batches that are spread over the GPU (full_slice_kernel): few rows, and bf16 ones that one
+// workgroup per row and CU takes in two rounds.  Measured, spread against whole rows (151936
+// ids, us a call): 128 rows fp32 52 and 60; 200 rows bf16 57 and 58, fp32 61 and 58; 256 rows
+// 71 and 60; 300 rows bf16 70 and 87, 400 rows 80 and 88; 500 rows fp32 109 and 90 (two
+// workgroups per CU).
 constexpr int PRE_MAX_ROWS = 128;
+constexpr int PRE_BF16_MIN = 257, PRE_BF16_MAX = 448;
+constexpr int PRE_GRID = 4096;  // workgroups wanted in all (128 rows fp32: 63 us at 512, 54 at 1024, 52 at 3072 or more)
 constexpr size_t PRE_MAX_LDS = 48 * 1024;  // a spread slice's history bitmap
 
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -168,6 +181,28 @@ struct Params {
   float* pre_em;
   uint64_t* pre_w;
   int32_t* pre_st;
+  // small top-p or min-p batch spread over the GPU (small_*_kernel): n_slices slices of slice_w
+  // ids a row, their partial results, and the row tables
+  struct SmallPart* sm_part;  // [rows, n_slices]
+  struct SmallRow* sm_row;    // [rows]
+  int32_t* sm_status;         // [rows]
+  int32_t* sm_count;          // [rows] tokens in sm_list
+  uint64_t* sm_list;          // [rows, TOPP_CAP]
+  uint64_t* sm_tables;        // [rows, TOPP_BINS + chunks] (top-p)
+};
+
+// What a slice of a row reports: its largest z and first index, later its mass, its kept tokens
+// and their exp sum; and what the row's boundary search found (top-p).
+struct SmallPart {
+  float mx;
+  int arg;
+  uint64_t tot;
+  double es;
+  int nk, pad;
+};
+struct SmallRow {
+  uint64_t thr, cum;
+  int bstar, pad;
 };
 
 // Per-workgroup scalars and reduction scratch, at the start of dynamic LDS.
@@ -541,7 +576,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const void* base, uin
   // gfx9 raw buffer: stride 0, num_records = bytes; reads past it return 0
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
 }
-
 // The bytes of a row of V logits that its buffer serves.  The range check of a vector load goes
 // dword by dword, so every id of a row that ends inside a vector is read; an odd bf16 row's last
 // id shares its dword with one element past the row, which every user masks by V.
@@ -3222,6 +3256,489 @@ __global__ __launch_bounds__(TOPK_NT) void merge_kernel(Params p, MergeIn in) {
   block_final<NT>(p, row, m, cand, n, hist);
 }
 
+// ====================================================================== small top-p / min-p
+// A batch of a few rows with top-p alone, or with min-p and no top-k, leaves most CUs idle with
+// one workgroup per row.  Its rows are then cut into slices of a few thousand ids, and the steps
+// that need the whole row (its maximum, its total mass and bins, its kept tokens) become launches
+// over all slices, each of which is a row of its own to the streaming code (as a vocabulary
+// shard is):
+//   small_max_kernel   every slice's largest z, first index and status; clears the row tables
+//   top-p:  small_bins_kernel  exact masses into the row total and (LDS, then global) bins
+//           small_keep_kernel  the boundary bin, the kept chunks' masses, its tokens
+//           small_topp_kernel  one workgroup per row: the boundary, the draw
+//   min-p:  small_minp_kernel  the tokens within the bound of the row maximum, to a list
+//           merge_kernel       the final selection over it
+// Every decision is the one topp_kernel or topk_kernel takes, on the same integers, so the ids and
+// kept sets are theirs.  Bound by the launches and their set-up at a few rows, by the masses and
+// bins at many.  A call of 48 bf16 rows with top-p 0.9 takes 134 us in topp_kernel and 72 here (8
+// fp32 rows 121 and 58, 128 rows 141 and 106); with min-p 0.05, 82 us in topk_kernel and 45 here.
+constexpr int SM_NT = 256;
+constexpr int SM_HR = 4;
+
+// This workgroup's slice as a row of its own; returns its first id.
+template <typename TIn>
+__device__ __forceinline__ int slice_of(Params& p, int& row, int& sl) {
+  row = (int)blockIdx.x / p.n_slices;
+  sl = (int)blockIdx.x % p.n_slices;
+  const int v0 = sl * p.slice_w;
+  p.voff = v0;
+  p.V = min(p.slice_w, p.vfull - v0);
+  p.logits = reinterpret_cast<const TIn*>(p.logits) + v0;
+  return v0;
+}
+
+// A slice's stream: tile(z, first id of the lane's G, t) for the stream's logits (history tokens
+// and the tail read -inf), hist(z, id) for the slice's history tokens; ids within the slice.
+template <typename TIn, bool VEC, int CPOL, class Init, class TileFn, class HistFn>
+__device__ __forceinline__ void slice_stream(const Params& p, int row, const Hist& h, Misc* m, int& bad, Init init,
+                                             TileFn tile, HistFn hist) {
+  constexpr int G = 4, NT = SM_NT, TILE = NT * G;
+  const int tid = threadIdx.x;
+  HistIds<SM_HR> hi;
+  load_history<NT, SM_HR>(p, row, hi);
+  const __amdgpu_buffer_rsrc_t rs = row_rsrc(row_ptr<TIn>(p, row), row_bytes<TIn>(p.V));
+  stream_row<TIn, G, NT, VEC, false, CPOL>(
+      p, rs, h,
+      [&]() {
+        if (tid == 0) m->status = 0;
+        init();
+        __syncthreads();
+        const int U = p.has_pen ? build_history<NT, SM_HR, true>(p, row, hi, h, m) : 0;
+        landed(hi);
+        return U;
+      },
+      [&](int t0, int nt, Raw<TIn, G>(&R)[PF], int s0, int n, float gx) {
+#pragma unroll
+        for (int k = 0; k < PF; ++k) {
+          const int t = t0 + k;
+          if (t < nt) {
+            const int base = t * TILE + tid * G;
+            float x[G], z[G];
+            unpack(R[k], x);
+            make_z<G, true>(x, base, p, h.bitmap, z, bad);
+            tile(z, base, t);
+          }
+        }
+        for (int i = tid; i < n; i += NT) {
+          const int s = s0 + i;
+          const int tok = (int)h.tok[s];
+          const float x = i == tid ? gx : load_one<TIn>(rs, tok);
+          const float z = pen_z(x, count_of(h, s), p);
+          if (!isfinite(z)) bad = 1;
+          hist(z, tok);
+        }
+      });
+}
+
+// The row maximum over its slices' (every lane of every wave gets it).
+__device__ __forceinline__ float small_row_max(const Params& p, int row) {
+  float mx = NEG_INF;
+  for (int s = threadIdx.x & 63; s < p.n_slices; s += 64) mx = fmaxf(mx, p.sm_part[row * p.n_slices + s].mx);
+  return wave_max_dpp(mx);
+}
+
+template <typename TIn, bool VEC>
+__global__ __launch_bounds__(SM_NT) void small_max_kernel(Params p) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int chunks = p.sm_tables ? n_chunks<4>(p.vfull) : 0;
+  int row, sl;
+  const int v0 = slice_of<TIn>(p, row, sl);
+  const Layout L = make_layout<MODE_GENERIC, 4>(p.V, p.words, p.ucap, 0);
+  Misc* m = reinterpret_cast<Misc*>(smem + L.misc);
+  const Hist h = hist_tables(smem, L);
+  const int tid = threadIdx.x;
+  if (p.sm_tables) {  // this slice's share of the row's tables
+    uint64_t* t = p.sm_tables + (int64_t)row * (TOPP_BINS + chunks);
+    for (int i = sl * SM_NT + tid; i < TOPP_BINS + chunks; i += p.n_slices * SM_NT) t[i] = 0;
+  }
+  if (sl == 0 && tid == 0) {
+    p.sm_count[row] = 0;
+    p.sm_status[row] = 0;
+  }
+  int bad = 0, bi = 0x7FFFFFFF;
+  float bm = NEG_INF;
+  slice_stream<TIn, VEC, 0>(
+      p, row, h, m, bad, []() {},
+      [&](const float (&z)[4], int base, int) {
+        if (!p.greedy) {  // (the index is a greedy draw's alone)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) bm = fmaxf(bm, z[j]);
+          return;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (z[j] > bm) {
+            bm = z[j];
+            bi = base + j;
+          }
+      },
+      [&](float z, int tok) {
+        if (z > bm || (z == bm && tok < bi)) {
+          bm = z;
+          bi = tok;
+        }
+      });
+  if (bad) atomicOr(&m->status, ST_NONFINITE);
+  const float mx = block_max<SM_NT>(bm, m);
+  const int arg = block_min_i<SM_NT>(bm == mx && bm > NEG_INF ? bi : 0x7FFFFFFF, m);
+  if (tid == 0) {
+    SmallPart& q = p.sm_part[row * p.n_slices + sl];
+    q.mx = mx;
+    q.arg = arg == 0x7FFFFFFF ? arg : arg + v0;
+    q.pad = m->status;
+  }
+}
+
+template <typename TIn, bool VEC>
+__global__ __launch_bounds__(SM_NT) void small_bins_kernel(Params p) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int V = p.vfull, chunks = n_chunks<4>(V);
+  int row, sl;
+  slice_of<TIn>(p, row, sl);
+  const Layout L = make_layout<MODE_GENERIC, 4>(p.V, p.words, p.ucap, 0);
+  Misc* m = reinterpret_cast<Misc*>(smem + L.misc);
+  const Hist h = hist_tables(smem, L);
+  uint64_t* bins = reinterpret_cast<uint64_t*>(smem + L.total);
+  const int tid = threadIdx.x;
+  const float zmax = small_row_max(p, row), dstar = topp_depth(p.top_p, V);
+  uint64_t tot = 0;
+  int bad = 0;
+  slice_stream<TIn, VEC, 0>(
+      p, row, h, m, bad,
+      [&]() {
+        for (int i = tid; i < TOPP_BINS; i += SM_NT) bins[i] = 0;
+      },
+      [&](const float (&z)[4], int, int) {
+        double ts = 0.0;  // (four masses of at most 2^43 sum exactly)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float ms = mass_ff(z[j], zmax);
+          ts += (double)ms;
+          if (z[j] - zmax >= dstar && ms != 0.0f)
+            atomicAdd((unsigned long long*)&bins[topp_bin(z[j], zmax)], (unsigned long long)ms);
+        }
+        tot += (uint64_t)ts;
+      },
+      [&](float z, int) {
+        const uint64_t ms = mass_of(z, zmax);
+        tot += ms;
+        if (z - zmax >= dstar && ms != 0)
+          atomicAdd((unsigned long long*)&bins[topp_bin(z, zmax)], (unsigned long long)ms);
+      });
+  tot = block_sum_u64<SM_NT>(tot, m);  // its barriers also order the bin atomics
+  if (tid == 0) p.sm_part[row * p.n_slices + sl].tot = tot;
+  uint64_t* g = p.sm_tables + (int64_t)row * (TOPP_BINS + chunks);
+  for (int i = tid; i < TOPP_BINS; i += SM_NT)
+    if (bins[i]) atomicAdd((unsigned long long*)&g[i], (unsigned long long)bins[i]);
+}
+
+template <typename TIn, bool VEC>
+__global__ __launch_bounds__(SM_NT) void small_keep_kernel(Params p) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int chunks = n_chunks<4>(p.vfull);
+  int row, sl;
+  const int v0 = slice_of<TIn>(p, row, sl);
+  const Layout L = make_layout<MODE_GENERIC, 4>(p.V, p.words, p.ucap, 0);
+  Misc* m = reinterpret_cast<Misc*>(smem + L.misc);
+  const Hist h = hist_tables(smem, L);
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  uint64_t* g = p.sm_tables + (int64_t)row * (TOPP_BINS + chunks);
+  uint64_t* gchunks = g + TOPP_BINS;
+  const float zmax = small_row_max(p, row);
+  uint64_t tot = 0;
+  for (int s = lane; s < p.n_slices; s += 64) tot += p.sm_part[row * p.n_slices + s].tot;
+  tot = wave_sum_u64(tot);
+  const uint64_t thr = top_p_threshold(p.top_p, tot);
+  // bin b* with (mass of bins < b*) < thr <= (mass of bins <= b*), as in topp_kernel: a run of
+  // bins per thread, in registers
+  constexpr int PER = TOPP_BINS / SM_NT;
+  uint64_t run[PER], own = 0;
+#pragma unroll
+  for (int q = 0; q < PER; ++q) {
+    run[q] = g[tid * PER + q];
+    own += run[q];
+  }
+  const uint64_t incl = wave_incl_scan_u64(own, lane);
+  if (tid == 0) m->bi[0] = -1;
+  if (lane == 63) m->ru[wid] = incl;
+  __syncthreads();
+  uint64_t before = incl - own;
+  for (int w = 0; w < wid; ++w) before += m->ru[w];
+  if (before < thr && thr <= before + own) {
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      if (before < thr && before + run[q] >= thr) {
+        m->bi[0] = tid * PER + q;
+        m->bu[0] = before;
+      }
+      before += run[q];
+    }
+  }
+  __syncthreads();
+  const int bstar = m->bi[0];
+  if (sl == 0 && tid == 0) {
+    SmallRow& r = p.sm_row[row];
+    r.thr = thr;
+    r.cum = m->bu[0];
+    r.bstar = bstar;
+  }
+  // tokens of bins up to b* have fl(zmax - z) below b*'s upper edge (the last bin has none)
+  const float edge = bstar < TOPP_BINS - 1 ? __uint_as_float((uint32_t)(bstar + TOPP_BIN_BASE + 1) << 16)
+                                           : __builtin_huge_valf();
+  const double dmax = (double)zmax;
+  double es = 0.0;
+  int nk = 0, bad = 0;
+  uint64_t* list = p.sm_list + (int64_t)row * TOPP_CAP;
+  auto boundary = [&](float z, int id) {
+    const int pos = atomicAdd(&p.sm_count[row], 1);
+    if (pos < TOPP_CAP) list[pos] = ckey(z, (uint32_t)id);
+  };
+  slice_stream<TIn, VEC, 0>(
+      p, row, h, m, bad, []() {},
+      [&](const float (&z)[4], int base, int) {
+        // A percent of the ids pass: each round takes every lane's next one, so a wave runs the
+        // 64-bit exp once or twice per tile and not once for each of a lane's four ids.
+        uint64_t cs = 0;
+        uint32_t left = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) left |= (uint32_t)(zmax - z[j] < edge) << j;
+        while (left) {
+          const int j = __ffs((int)left) - 1;
+          left &= left - 1;
+          const float zj = j < 2 ? (j == 0 ? z[0] : z[1]) : (j == 2 ? z[2] : z[3]);
+          const double d = (double)zj - dmax;
+          if (d >= -30.0) {
+            const int b = topp_bin(zj, zmax);
+            if (b < bstar) {
+              cs += mass_of(zj, zmax);
+              es += exp_det(d);
+              ++nk;
+            } else if (b == bstar) {
+              boundary(zj, v0 + base + j);
+            }
+          }
+        }
+        if (__ballot(cs != 0)) {  // (a wave's 256 ids of a tile are one chunk)
+          cs = wave_sum_u64(cs);
+          if (lane == 0) atomicAdd((unsigned long long*)&gchunks[(v0 + base) >> 8], (unsigned long long)cs);
+        }
+      },
+      [&](float z, int tok) {
+        const double d = (double)z - dmax;
+        if (d >= -30.0) {
+          const int b = topp_bin(z, zmax);
+          if (b < bstar) {
+            atomicAdd((unsigned long long*)&gchunks[(v0 + tok) >> 8], (unsigned long long)mass_of(z, zmax));
+            es += exp_det(d);
+            ++nk;
+          } else if (b == bstar) {
+            boundary(z, v0 + tok);
+          }
+        }
+      });
+  nk = block_sum_i<SM_NT>(nk, m);
+  es = block_sum_d<SM_NT>(es, m);
+  if (tid == 0) {
+    SmallPart& q = p.sm_part[row * p.n_slices + sl];
+    q.nk = nk;
+    q.es = es;
+  }
+}
+
+// One workgroup per row: the boundary inside bin b*, the kept set's sums and the draw.
+constexpr int SM_FIN_NT = 512;
+__host__ __device__ inline size_t small_fin_tables(int ucap) {  // Misc, history of one chunk
+  return make_layout<MODE_GENERIC, 4>(256, 8, ucap < 256 ? ucap : 256, 0).total;
+}
+template <typename TIn>
+__global__ __launch_bounds__(SM_FIN_NT) void small_topp_kernel(Params p) {
+  constexpr int NT = SM_FIN_NT;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int V = p.V, chunks = n_chunks<4>(V);
+  const int slices = p.n_slices;
+  Params q = p;  // (the chunk that is read again, as a row of its own)
+  q.words = p.has_pen ? 8 : 0;
+  q.ucap = min(p.ucap, 256);
+  const Layout L = make_layout<MODE_GENERIC, 4>(256, q.words, q.ucap, 0);
+  Misc* m = reinterpret_cast<Misc*>(smem + L.misc);
+  const Hist h = hist_tables(smem, L);
+  uint64_t* ch = reinterpret_cast<uint64_t*>(smem + small_fin_tables(p.ucap));
+  uint64_t* blist = ch + chunks;
+  const uint64_t* g = p.sm_tables + (int64_t)row * (TOPP_BINS + chunks) + TOPP_BINS;
+  const SmallRow r = p.sm_row[row];
+  const int nc = p.sm_count[row];
+  HistIds<SM_HR> hi;
+  load_history<NT, SM_HR>(p, row, hi);
+  if (tid == 0) m->status = 0;
+  __syncthreads();
+  // the slices' results in slice order
+  float bm = NEG_INF;
+  int st = 0, am = 0x7FFFFFFF, nk = 0;
+  double es = 0.0;
+  for (int s = tid; s < slices; s += NT) {
+    const SmallPart& part = p.sm_part[row * slices + s];
+    if (part.mx > bm) {
+      bm = part.mx;
+      am = part.arg;
+    }
+    st |= part.pad;
+    nk += part.nk;
+    es += part.es;
+  }
+  if (st) atomicOr(&m->status, st);
+  const float zmax = block_max<NT>(bm, m);
+  am = block_min_i<NT>(bm == zmax ? am : 0x7FFFFFFF, m);
+  if (am < 0 || am >= V) am = 0;
+  const float u = row_uniform(p, row, m);
+  __syncthreads();
+  if (m->status & ST_NONFINITE) {
+    if (tid == 0) write_result(p, row, m, am, 0.0f, 0);
+    return;
+  }
+  if (nc > TOPP_CAP || nc < 1 || r.bstar < 0) {
+    if (tid == 0) p.out_status[row] = m->status | ST_FALLBACK;
+    return;
+  }
+  for (int i = tid; i < chunks; i += NT) ch[i] = g[i];
+  for (int i = tid; i < nc; i += NT) blist[i] = p.sm_list[(int64_t)row * TOPP_CAP + i];
+  __syncthreads();
+  if (nc <= 64) {
+    if (wid == 0) {
+      const uint64_t key = wave_rank_desc(lane < nc ? blist[lane] : 0, blist, nc, lane);
+      (void)key;
+    }
+    __syncthreads();
+  } else {
+    bitonic_sort_desc<NT>(blist, nc);
+    __syncthreads();
+  }
+  if (wid == 0) {
+    uint64_t carry = r.cum;
+    int js = nc - 1;
+    for (int c0 = 0; c0 < nc; c0 += 64) {
+      const int j = c0 + lane;
+      const uint64_t ms = j < nc ? mass_of(ckey_z(blist[j]), zmax) : 0;
+      const uint64_t incl = wave_incl_scan_u64(ms, lane) + carry;
+      const uint64_t hit = __builtin_amdgcn_ballot_w64(j < nc && incl >= r.thr);
+      if (hit) {
+        js = c0 + __builtin_ctzll(hit);
+        break;
+      }
+      carry = __shfl(incl, 63);
+    }
+    if (lane == 0) m->bi[1] = js;
+  }
+  __syncthreads();
+  const int jstar = m->bi[1];
+  for (int j = tid; j <= jstar; j += NT) {
+    const uint64_t key = blist[j];
+    atomicAdd((unsigned long long*)&ch[ckey_idx(key) >> 8], (unsigned long long)mass_of(ckey_z(key), zmax));
+    es += exp_det((double)ckey_z(key) - (double)zmax);
+    ++nk;
+  }
+  const uint64_t Bkey = blist[jstar];
+  nk = block_sum_i<NT>(nk, m);
+  const double esum = block_sum_d<NT>(es, m);  // its barriers also order the chunk atomics
+  int64_t tok = am;
+  float ztok = zmax;
+  if (!p.greedy) {
+    uint64_t sk = 0;
+    for (int i = tid; i < chunks; i += NT) sk += ch[i];
+    sk = block_sum_u64<NT>(sk, m);
+    const uint64_t t = draw_target(u, sk);
+    block_incl_scan_u64<NT>(ch, chunks, m);
+    for (int c = tid; c < chunks; c += NT) {
+      const uint64_t before = c ? ch[c - 1] : 0;
+      if (before <= t && t < ch[c]) {
+        m->bi[2] = c;
+        m->bu[1] = before;
+      }
+    }
+    __syncthreads();
+    const int c = m->bi[2];
+    const uint64_t before = m->bu[1];
+    q.voff = c * 256;
+    q.V = min(256, V - q.voff);
+    if (p.has_pen) build_history<NT, SM_HR, true>(q, row, hi, h, m);
+    landed(hi);
+    if (wid == 0) {
+      const __amdgpu_buffer_rsrc_t rs = row_rsrc(row_ptr<TIn>(p, row), row_bytes<TIn>(V));
+      uint64_t ms[4], ls = 0;
+      float zz[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = lane * 4 + j, idx = q.voff + i;
+        float z = NEG_INF;
+        if (idx < V) {
+          const float x = load_one<TIn>(rs, idx);
+          if (p.has_pen && ((h.bitmap[i >> 5] >> (i & 31)) & 1u)) z = pen_z(x, count_of(h, slot_of(h, i)), p);
+          else z = div_T(x, p);
+        }
+        zz[j] = z;
+        ms[j] = 0;
+        if ((double)z - (double)zmax >= -30.0 && ckey(z, (uint32_t)idx) >= Bkey) ms[j] = mass_of(z, zmax);
+        ls += ms[j];
+      }
+      uint64_t acc = wave_incl_scan_u64(ls, lane) + before - ls;
+      int pick = -1;
+      float zp = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (pick < 0 && ms[j] != 0 && t < acc + ms[j]) {
+          pick = q.voff + lane * 4 + j;
+          zp = zz[j];
+        }
+        acc += ms[j];
+      }
+      const uint64_t hit = __builtin_amdgcn_ballot_w64(pick >= 0);
+      if (hit) {
+        const int src_lane = __builtin_ctzll(hit);
+        tok = __shfl(pick, src_lane);
+        ztok = __shfl(zp, src_lane);
+      }
+    }
+  }
+  if (tid == 0) {
+    const float lp = (float)(((double)ztok - (double)zmax) - log(esum));
+    write_result(p, row, m, tok, lp, nk);
+  }
+}
+
+template <typename TIn, bool VEC>
+__global__ __launch_bounds__(SM_NT) void small_minp_kernel(Params p) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  int row, sl;
+  const int v0 = slice_of<TIn>(p, row, sl);
+  const Layout L = make_layout<MODE_GENERIC, 4>(p.V, p.words, p.ucap, 0);
+  Misc* m = reinterpret_cast<Misc*>(smem + L.misc);
+  const Hist h = hist_tables(smem, L);
+  const float zmax = small_row_max(p, row);
+  const float bnd = minp_bound_f(zmax, p.lmin_f);  // at or below the exact bound
+  uint64_t* list = p.sm_list + (int64_t)row * TOPP_CAP;
+  int bad = 0;
+  auto offer = [&](float z, int id) {
+    if (z > NEG_INF && z >= bnd && minp_ok(z, zmax, p)) {
+      const int pos = atomicAdd(&p.sm_count[row], 1);
+      if (pos < TOPP_CAP) list[pos] = ckey(z, (uint32_t)(v0 + id));
+      else atomicOr(&p.sm_status[row], ST_FALLBACK);
+    }
+  };
+  if (sl == 0 && threadIdx.x < 64) {  // the row's status so far, from its slices
+    int st = 0;
+    for (int s = threadIdx.x; s < p.n_slices; s += 64) st |= p.sm_part[row * p.n_slices + s].pad;
+    for (int o = 32; o > 0; o >>= 1) st |= __shfl_xor(st, o);
+    if (threadIdx.x == 0 && st) atomicOr(&p.sm_status[row], st);
+  }
+  slice_stream<TIn, VEC, 0>(
+      p, row, h, m, bad, []() {},
+      [&](const float (&z)[4], int base, int) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) offer(z[j], base + j);
+      },
+      [&](float z, int tok) { offer(z, tok); });
+}
+
 // One thread per row of a full-vocabulary draw over slices: the row's maximum and total
 // from the gathered states, the token from the picks (inverse CDF: the one slice that
 // placed it; race: the best p / E, first id on ties; greedy: the first slice holding the
@@ -3309,7 +3826,8 @@ struct Plan {
                     // (TOPP rows fall back to generic_kernel the same way)
   int words, ucap, cap;
   size_t lds;
-  size_t workspace;
+  size_t workspace;   // bytes wanted, and those without which the batch is refused; with fewer
+  size_t required;    // than wanted a FULL batch is not spread
   int topk_nt;        // TOPK threads per workgroup: TOPK_NT, or 256 (see plan)
   int topp_nt;        // TOPP threads per workgroup: TOPP_NT, or 512 (see plan)
   bool bitmap_only;   // TOPK penalties need only the membership bitmap
@@ -3322,6 +3840,10 @@ struct Plan {
   // of its arrays
   int pre_slices, pre_sw;
   size_t pre_lds, pre_em, pre_w, pre_st;
+  // small top-p or min-p batch over sm_slices slices of slice_w ids per row (0: none), with the
+  // LDS of a slice and of the finish and the workspace offsets of its arrays
+  int sm_slices;
+  size_t sm_lds, sm_fin_lds, sm_row, sm_status, sm_count, sm_list, sm_tables;
 };
 
 // shard: the descriptor describes one vocabulary slice (dsv41_sampler_shard_run); the draw
@@ -3410,7 +3932,7 @@ int plan(const dsv41_sampler_desc* d, Plan* pl, bool shard = false) {
   pl->defer = !shard && pl->mode == MODE_TOPK && d->rows > DEFER_MIN_ROWS;
   // Batches of at least two rows per CU whose TOPP tables fit two workgroups per CU run
   // with 512 threads: a row's first read (memory) then overlaps another's mass pass (ALU).
-  pl->topp_nt = pl->mode == MODE_TOPP && d->rows >= 512 && 2 * pl->lds <= LDS_LIMIT ? 512 : TOPP_NT;
+  pl->topp_nt = pl->mode == MODE_TOPP && d->rows > 256 && 2 * pl->lds <= LDS_LIMIT ? 512 : TOPP_NT;
   // Deferred TOPK batches whose tables fit four 256-thread workgroups per CU (a quarter of
   // LDS) run with 256 threads: 128 VGPRs then hold four rows per CU instead of two, so a
   // row building its history tables leaves three others streaming.  Lowering penalties
@@ -3462,16 +3984,18 @@ int plan(const dsv41_sampler_desc* d, Plan* pl, bool shard = false) {
       }
     }
   }
-  // A FULL batch of at most PRE_MAX_ROWS rows leaves most CUs idle with one workgroup per
-  // row: about 512 workgroups then each take a run of a row's wave spans (full_slice_kernel,
+  // A FULL batch of few rows leaves most CUs idle with one workgroup per row: about PRE_GRID
+  // workgroups then each take a run of a row's wave spans (full_slice_kernel,
   // with its range's history bitmap in LDS), and one workgroup per row finishes it from
   // their statistics.
   pl->pre_slices = 0;
   pl->pre_lds = 0;
-  if (!shard && pl->mode == MODE_FULL && !d->replay_ids && !d->exponentials && d->rows <= PRE_MAX_ROWS) {
+  pl->required = pl->workspace;
+  if (!shard && pl->mode == MODE_FULL && !d->exponentials &&
+      (d->rows <= PRE_MAX_ROWS || (pl->esize == 2 && d->rows >= PRE_BF16_MIN && d->rows <= PRE_BF16_MAX))) {
     const int G = pl->esize == 4 ? 4 : 8;  // the spread small batches take 4 fp32 logits per lane
     const int NC = (V + 64 * G - 1) / (64 * G), NE = n_mass_chunks(V);
-    const int want = std::max(2, 512 / d->rows);
+    const int want = std::max(2, PRE_GRID / d->rows);
     const int sw = std::max(PRE_NT / 64, (NC + want - 1) / want);  // at least one span per wave
     const int S = (NC + sw - 1) / sw;
     const size_t slds = pl->has_pen ? (size_t)sw * 2 * G * sizeof(uint32_t) : 0;
@@ -3486,14 +4010,54 @@ int plan(const dsv41_sampler_desc* d, Plan* pl, bool shard = false) {
       off = align16(off + (size_t)d->rows * NE * sizeof(uint64_t));
       pl->pre_st = off;
       pl->workspace = off + (size_t)d->rows * S * sizeof(int32_t);
+      // replays and the larger batches ran without a workspace before: they still may
+      if (!d->replay_ids && d->rows <= PRE_MAX_ROWS) pl->required = pl->workspace;
     }
+  } else {
+    pl->required = pl->workspace;
   }
   if (pl->mode == MODE_GENERIC || pl->mode == MODE_TOPP || pl->internal_k) {
     pl->workspace = align16(pl->workspace);  // the z rows follow the hand-over area
     pl->workspace += (size_t)d->rows * (size_t)V * sizeof(float);
+    pl->required = pl->workspace;
     Layout Lg = make_layout<MODE_GENERIC, 4>(V, pl->words, pl->ucap, 0);
     if (Lg.total > LDS_LIMIT)
       return fail(DSV41_E_UNSUPPORTED, "history length and vocabulary exceed the on-chip penalty tables");
+  }
+  // Top-p alone, or min-p without top-k, on few rows: slices of at least SMALL_MIN_W ids.  Their tables lie in the z rows of the fallback, which
+  // runs after them.
+  pl->sm_slices = 0;
+  const bool topp = pl->mode == MODE_TOPP;
+  if (!shard && (topp || pl->internal_k) && d->rows <= (topp ? SMALL_TOPP_ROWS : SMALL_MINP_ROWS) && V >= 4 * SMALL_MIN_W) {
+    const int want = std::max(1, (topp ? SMALL_TOPP_GRID : SMALL_MINP_GRID) / d->rows);
+    const int tile = SM_NT * 4;
+    const int sw = std::max(SMALL_MIN_W, ((V + want - 1) / want + tile - 1) / tile * tile);
+    const int S = (V + sw - 1) / sw, chunks = n_chunks<4>(V);
+    const int words = pl->has_pen ? (sw + 31) / 32 : 0;
+    const int ucap = pl->has_pen ? (int)std::min<int64_t>(d->history_row_stride, sw) : 0;
+    const size_t lds = make_layout<MODE_GENERIC, 4>(sw, words, ucap, 0).total;
+    const size_t fin = small_fin_tables(pl->has_pen ? (int)std::min<int64_t>(d->history_row_stride, V) : 0) +
+                       ((size_t)chunks + TOPP_CAP) * sizeof(uint64_t);
+    const size_t n = (size_t)d->rows;
+    size_t off = n * S * sizeof(SmallPart);
+    pl->sm_row = off;
+    off += n * sizeof(SmallRow);
+    pl->sm_list = off;
+    off += n * TOPP_CAP * sizeof(uint64_t);
+    pl->sm_tables = off;
+    off += topp ? n * (TOPP_BINS + chunks) * sizeof(uint64_t) : 0;
+    pl->sm_status = off;
+    off += n * sizeof(int32_t);
+    pl->sm_count = off;
+    off += n * sizeof(int32_t);
+    if (S >= 2 && lds + (topp ? TOPP_BINS * sizeof(uint64_t) : 0) <= SMALL_MAX_LDS && fin <= LDS_LIMIT && off <= pl->workspace) {
+      pl->sm_slices = S;
+      pl->slice_w = sw;
+      pl->slice_words = words;
+      pl->slice_ucap = ucap;
+      pl->sm_lds = lds;
+      pl->sm_fin_lds = fin;
+    }
   }
   return DSV41_OK;
 }
@@ -3688,6 +4252,12 @@ static int run_presliced(const dsv41_sampler_desc* d, const Plan& pl, const Para
     }
   }
   DSV41_HIP_CHECK(hipGetLastError());
+  if (p.replay) {
+    if (bf) return pl.vec ? launch(full_kernel<uint16_t, 8, true, DRAW_REPLAY, true>, FULL_NT, pl.lds, d->rows, p, s)
+                          : launch(full_kernel<uint16_t, 8, false, DRAW_REPLAY, true>, FULL_NT, pl.lds, d->rows, p, s);
+    return pl.vec ? launch(full_kernel<float, 4, true, DRAW_REPLAY, true>, FULL_NT, pl.lds, d->rows, p, s)
+                  : launch(full_kernel<float, 4, false, DRAW_REPLAY, true>, FULL_NT, pl.lds, d->rows, p, s);
+  }
   if (bf) {
     if (ex) return pl.vec ? launch(full_kernel<uint16_t, 8, true, DRAW_CDF, true>, FULL_NT, pl.lds, d->rows, p, s)
                           : launch(full_kernel<uint16_t, 8, false, DRAW_CDF, true>, FULL_NT, pl.lds, d->rows, p, s);
@@ -3704,12 +4274,59 @@ static int run_presliced(const dsv41_sampler_desc* d, const Plan& pl, const Para
                 : launch(full_kernel<float, 4, false, DRAW_GREEDY, true>, FULL_NT, pl.lds, d->rows, p, s);
 }
 
+// A small top-p or min-p batch: the slices' launches, then one finishing workgroup per row.
+template <typename TIn, bool VEC>
+static int run_small(const dsv41_sampler_desc* d, const Plan& pl, const Params& p, char* ws, hipStream_t s) {
+  Params q = p;
+  q.words = pl.slice_words;
+  q.ucap = pl.slice_ucap;
+  q.vfull = d->vocab;
+  q.n_slices = pl.sm_slices;
+  q.slice_w = pl.slice_w;
+  q.sm_part = reinterpret_cast<SmallPart*>(ws);
+  q.sm_row = reinterpret_cast<SmallRow*>(ws + pl.sm_row);
+  q.sm_status = reinterpret_cast<int32_t*>(ws + pl.sm_status);
+  q.sm_count = reinterpret_cast<int32_t*>(ws + pl.sm_count);
+  q.sm_list = reinterpret_cast<uint64_t*>(ws + pl.sm_list);
+  const bool topp = pl.mode == MODE_TOPP;
+  q.sm_tables = topp ? reinterpret_cast<uint64_t*>(ws + pl.sm_tables) : nullptr;
+  const int grid = d->rows * pl.sm_slices;
+  int rc = launch(small_max_kernel<TIn, VEC>, SM_NT, pl.sm_lds, grid, q, s);
+  if (rc != DSV41_OK) return rc;
+  if (topp) {
+    rc = launch(small_bins_kernel<TIn, VEC>, SM_NT, pl.sm_lds + TOPP_BINS * sizeof(uint64_t), grid, q, s);
+    if (rc != DSV41_OK) return rc;
+    rc = launch(small_keep_kernel<TIn, VEC>, SM_NT, pl.sm_lds, grid, q, s);
+    if (rc != DSV41_OK) return rc;
+    q.ucap = pl.ucap;
+    rc = launch(small_topp_kernel<TIn>, SM_FIN_NT, pl.sm_fin_lds, d->rows, q, s);
+    return rc;
+  }
+  rc = launch(small_minp_kernel<TIn, VEC>, SM_NT, pl.sm_lds, grid, q, s);
+  if (rc != DSV41_OK) return rc;
+  Params m = p;
+  m.top_k = TOPP_CAP;
+  m.topk_internal = 0;
+  MergeIn in{q.sm_list, q.sm_count, q.sm_status, 1, d->rows, TOPP_CAP, TOPP_CAP};
+  DSV41_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(merge_kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_LIMIT));
+  hipLaunchKernelGGL(merge_kernel, dim3(d->rows), dim3(TOPK_NT), merge_lds_bytes(TOPP_CAP, TOPP_CAP), s, m, in);
+  DSV41_HIP_CHECK(hipGetLastError());
+  return DSV41_OK;
+}
+
 // The launches of one planned batch; `workspace` holds at least pl.workspace bytes.
 static int run_planned(const dsv41_sampler_desc* d, const Plan& pl, void* workspace, void* stream) {
   int rc;
   Params p = make_params(d, pl, workspace);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool bf = pl.esize == 2;
+  if (pl.sm_slices) {
+    char* ws = static_cast<char*>(workspace);
+    if (bf) rc = pl.vec ? run_small<uint16_t, true>(d, pl, p, ws, s) : run_small<uint16_t, false>(d, pl, p, ws, s);
+    else rc = pl.vec ? run_small<float, true>(d, pl, p, ws, s) : run_small<float, false>(d, pl, p, ws, s);
+    return rc != DSV41_OK ? rc : run_flagged(d, pl, p, s);
+  }
   switch (pl.mode) {
     case MODE_FULL:
       if (pl.pre_slices) return run_presliced(d, pl, p, s);
@@ -3797,8 +4414,11 @@ extern "C" int dsv41_sampler_run(const dsv41_sampler_desc* d, void* workspace, s
   Plan pl;
   const int rc = plan(d, &pl);
   if (rc != DSV41_OK) return rc;
-  if (pl.workspace && (!workspace || workspace_bytes < pl.workspace))
-    return fail(DSV41_E_WORKSPACE, "sampler workspace is missing or too small");
+  if (pl.workspace && (!workspace || workspace_bytes < pl.workspace)) {
+    if (pl.required && (!workspace || workspace_bytes < pl.required))
+      return fail(DSV41_E_WORKSPACE, "sampler workspace is missing or too small");
+    pl.pre_slices = 0;
+  }
   return run_planned(d, pl, workspace, stream);
 }
 
@@ -3840,8 +4460,9 @@ extern "C" int dsv41_sampler_run_static(const dsv41_sampler_desc* d, void* strea
   Plan pl;
   int rc = plan(d, &pl);
   if (rc != DSV41_OK) return rc;
-  if (pl.workspace > (size_t)DSV41_SAMPLER_STATIC_SCRATCH_BYTES)
-    return fail(DSV41_E_UNSUPPORTED, "this batch needs " + std::to_string(pl.workspace) +
+  if (pl.workspace > (size_t)DSV41_SAMPLER_STATIC_SCRATCH_BYTES) pl.pre_slices = 0;
+  if (pl.required > (size_t)DSV41_SAMPLER_STATIC_SCRATCH_BYTES)
+    return fail(DSV41_E_UNSUPPORTED, "this batch needs " + std::to_string(pl.required) +
                                          " bytes of scratch, above the static maximum of " +
                                          std::to_string((size_t)DSV41_SAMPLER_STATIC_SCRATCH_BYTES) +
                                          " (use dsv41_sampler_run with a workspace)");

@@ -692,9 +692,11 @@ def replay_log_probs(
     desc.replay_ids = token_ids.data_ptr()
     desc.out_ids, desc.out_logprob, desc.out_status = ids.data_ptr(), lps.data_ptr(), status.data_ptr()
     lib = _lib.load()
+    ws_bytes = lib.dsv41_sampler_workspace_bytes(_lib.ctypes.byref(desc))
+    workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes else None
     with torch.cuda.device(device):
         stream = torch.cuda.current_stream(device).cuda_stream
-        rc = lib.dsv41_sampler_run(_lib.ctypes.byref(desc), None, 0, stream)
+        rc = lib.dsv41_sampler_run(_lib.ctypes.byref(desc), _device_ptr(workspace), ws_bytes, stream)
     _lib.check(rc)
     if check:
         if any_set(status)[0]:
