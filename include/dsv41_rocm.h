@@ -330,7 +330,7 @@ typedef struct dsv41_logprob_combine_desc {
  * with lse and entropy as written by dsv41_logprob_run.  NULL grad_logprob or grad_entropy
  * counts as zero.  The logits are recomputed on the matrix cores, never stored in fp32.
  * dL/dx = out @ w[vocab_begin:vocab_end] and dL/dw[vocab_begin:vocab_end] = out^T @ x are
- * plain GEMMs left to the caller's BLAS.
+ * dsv41_head_dx_run and dsv41_head_dw_run.
  */
 typedef struct dsv41_logprob_grad_desc {
   uint32_t struct_size; /* = sizeof(dsv41_logprob_grad_desc) */
@@ -543,6 +543,19 @@ int dsv41_logprob_combine_run(const dsv41_logprob_combine_desc* desc, void* stre
 
 /* Gradient of the fused log-prob with respect to the logits (no workspace). */
 int dsv41_logprob_grad_run(const dsv41_logprob_grad_desc* desc, void* stream /* hipStream_t */);
+
+/* The products of the head's backward with that gradient g [n, v] (row stride gs; the columns up to
+ * the next multiple of 8 must hold finite values): dx[n, h] = sum_v g w with w [v, h], and
+ * dw[v, h] = sum_n g x with x [n, h], operands bf16, sums fp32.  Strides in elements, multiples of
+ * 8; pointers 16-byte aligned; h a multiple of 8.  out_mode: 0 writes dx in bf16, 1 in fp32, 2
+ * adds it to an fp32 dx (vocabulary ranges in turn); dx rows are h elements apart.  The
+ * workspace serves mode 0.  They stand for the two GEMMs of nn.Linear's backward
+ * (distributed_grpo.py:352-375 over native_lora.py:120-122). */
+size_t dsv41_head_dx_workspace_bytes(int n, int v, int h);
+int dsv41_head_dx_run(const void* g, int64_t gs, const void* w, int64_t ws, int n, int v, int h, void* out,
+                      int out_mode, void* workspace, size_t workspace_bytes, void* stream /* hipStream_t */);
+int dsv41_head_dw_run(const void* g, int64_t gs, const void* x, int64_t xs, int n, int v, int h, void* out,
+                      int64_t out_row_stride, void* stream /* hipStream_t */);
 
 /* Token-TIS loss, gradient and metrics: replaces algorithm.py:249-346 for a batch of
  * responses, pooled as distributed_grpo.py:197-222. */

@@ -313,6 +313,9 @@ EXPORTS = (
     "dsv41_sampler_full_draw_run",
     "dsv41_sampler_full_finish_run",
     "dsv41_check_wait",
+    "dsv41_head_dx_workspace_bytes",
+    "dsv41_head_dx_run",
+    "dsv41_head_dw_run",
 )
 
 _lock = threading.Lock()
@@ -372,6 +375,15 @@ def _bind(lib: ctypes.CDLL) -> ctypes.CDLL:
         getattr(lib, name).argtypes = [ctypes.POINTER(SamplerFullShardDesc), ctypes.c_void_p]
     lib.dsv41_sampler_full_finish_run.restype = ctypes.c_int
     lib.dsv41_sampler_full_finish_run.argtypes = [ctypes.POINTER(SamplerFullFinishDesc), ctypes.c_void_p]
+    lib.dsv41_head_dx_workspace_bytes.restype = ctypes.c_size_t
+    lib.dsv41_head_dx_workspace_bytes.argtypes = [ctypes.c_int] * 3
+    lib.dsv41_head_dx_run.restype = ctypes.c_int
+    lib.dsv41_head_dx_run.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int,
+                                      ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p,
+                                      ctypes.c_size_t, ctypes.c_void_p]
+    lib.dsv41_head_dw_run.restype = ctypes.c_int
+    lib.dsv41_head_dw_run.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int,
+                                      ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
     lib.dsv41_check_wait.restype = ctypes.c_int
     lib.dsv41_check_wait.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64,
                                     ctypes.c_void_p, ctypes.c_void_p]

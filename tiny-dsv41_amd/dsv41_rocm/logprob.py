@@ -17,7 +17,7 @@ from the bf16 operands (the reference rounds ``lm_head``'s output to bf16 first)
 Under autograd the head is differentiable as the reference's is when the learner scores
 its ``current`` phase (``dsv41_train/rl/distributed_grpo.py:352-375`` through the
 checkpointed ``_score_targets``, ``native_lora.py:120-122``): the backward recomputes the
-logits tile by tile and produces their gradient in bf16, then takes the two GEMMs.
+logits tile by tile and produces their gradient in bf16, then takes the two products with it.
 """
 
 from __future__ import annotations
@@ -127,6 +127,8 @@ def logits_grad(hidden: torch.Tensor, weight: torch.Tensor, targets: torch.Tenso
     width = vocab_end - vocab_begin
     stride = (width + 7) // 8 * 8
     out = torch.empty(n, stride, dtype=torch.bfloat16, device=hidden.device)
+    if stride != width:
+        out[:, width:].zero_()  # the products read whole 16-byte chunks of a row
     f32 = lambda t: None if t is None else t.to(device=hidden.device, dtype=torch.float32).reshape(-1).contiguous()
     lse, entropy, grad_logprob, grad_entropy = f32(lse), f32(entropy), f32(grad_logprob), f32(grad_entropy)
     d = _lib.LogprobGradDesc()
@@ -155,6 +157,10 @@ def logits_grad(hidden: torch.Tensor, weight: torch.Tensor, targets: torch.Tenso
 # = 1.06 GB); at 16384 tokens x 129280 rows it takes four ranges of 32768 rows.
 GRAD_BLOCK_BYTES = 1 << 30
 
+# dL/dweight of fewer tokens than this is a write of the weights and little else, which the library
+# GEMM does faster (7168 x 129280: 32 tokens 0.46 ms against 0.53; 300 tokens 1.09 against 0.93).
+DW_MIN_TOKENS = 96
+
 
 def selected_log_probs_backward(hidden, weight, targets, temperature, lse, entropy, grad_logprob,
                                 grad_entropy, need_hidden=True, need_weight=True, vocab_chunk=None):
@@ -162,27 +168,37 @@ def selected_log_probs_backward(hidden, weight, targets, temperature, lse, entro
 
     The logit gradient comes from ``dsv41_logprob_grad_run`` (recomputed logits on the
     matrix cores, bf16 like the reference's ``lm_head`` output gradient); the two products
-    with it are plain GEMMs (hipBLASLt through torch), as in the reference's ``nn.Linear``
-    backward.  Vocabulary ranges of ``vocab_chunk`` rows (default: as many as
+    with it, the reference's ``nn.Linear`` backward, are ``dsv41_head_dx_run`` and
+    ``dsv41_head_dw_run``.  Vocabulary ranges of ``vocab_chunk`` rows (default: as many as
     ``GRAD_BLOCK_BYTES`` allows) bound the logit gradient held at once.
     """
-    n, _ = hidden.shape
+    n, h = hidden.shape
     v = weight.shape[0]
+    if n == 0:
+        return (torch.zeros_like(hidden) if need_hidden else None), (torch.zeros_like(weight) if need_weight else None)
     if vocab_chunk is None:
         vocab_chunk = max(256, GRAD_BLOCK_BYTES // max(1, 2 * n) // 256 * 256)
     ranges = [(b, min(v, b + vocab_chunk)) for b in range(0, v, vocab_chunk)]
-    dx = None
+    # one range writes dx in bf16; several add up in fp32
+    whole = len(ranges) == 1
+    dx = torch.empty(n, h, dtype=hidden.dtype if whole else torch.float32, device=hidden.device) if need_hidden else None
     dw = torch.empty_like(weight) if need_weight else None
+    lib = _lib.load()
     for b, e in ranges:
         g = logits_grad(hidden, weight, targets, temperature, lse, entropy, grad_logprob, grad_entropy, b, e)
-        if need_hidden:
-            part = torch.mm(g, weight[b:e])
-            if len(ranges) == 1:
-                dx = part
-            else:
-                dx = part.float() if dx is None else dx.add_(part.float())
-        if need_weight:
-            torch.mm(g.t(), hidden, out=dw[b:e])
+        with torch.cuda.device(hidden.device):
+            stream = torch.cuda.current_stream(hidden.device).cuda_stream
+            if need_hidden:
+                ws_bytes = lib.dsv41_head_dx_workspace_bytes(n, e - b, h) if whole else 0
+                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=hidden.device) if ws_bytes else None
+                _lib.check(lib.dsv41_head_dx_run(g.data_ptr(), g.stride(0), weight[b:e].data_ptr(), weight.stride(0), n,
+                                                 e - b, h, dx.data_ptr(), 0 if whole else (1 if b == 0 else 2),
+                                                 ws.data_ptr() if ws_bytes else None, ws_bytes, stream))
+            if need_weight and n < DW_MIN_TOKENS:
+                torch.mm(g.t(), hidden, out=dw[b:e])
+            elif need_weight:
+                _lib.check(lib.dsv41_head_dw_run(g.data_ptr(), g.stride(0), hidden.data_ptr(), hidden.stride(0), n,
+                                                 e - b, h, dw[b:e].data_ptr(), dw.stride(0), stream))
     if dx is not None:
         dx = dx.to(hidden.dtype)
     return dx, dw
@@ -190,7 +206,7 @@ def selected_log_probs_backward(hidden, weight, targets, temperature, lse, entro
 
 class _SelectedLogProbs(torch.autograd.Function):
     """Differentiable fused log-prob: forward = dsv41_logprob_run, backward =
-    dsv41_logprob_grad_run + two GEMMs.  The Token-TIS weight carries no gradient (the
+    dsv41_logprob_grad_run + the two products.  The Token-TIS weight carries no gradient (the
     reference computes it from detached old log-probs, algorithm.py:293-299)."""
 
     @staticmethod
