@@ -409,7 +409,7 @@ def bench_logprob(name, steps, warmup, cpu_baseline, torch, backward=False):
 def bench_logprob_backward(x, w, t, lp, ent, steps, torch):
     """Backward of the fused log-prob for dL/dlogprob = 1 per token: the logit-gradient
     kernel (logits recomputed on MFMA, bf16 gradient written once) and the whole backward
-    with the two GEMMs (hipBLASLt through torch) that produce dL/dx and dL/dw."""
+    with the two products that give dL/dx and dL/dw."""
     from dsv41_rocm import logprob as lpmod
 
     n, h = x.shape
@@ -434,7 +434,7 @@ def bench_logprob_backward(x, w, t, lp, ent, steps, torch):
                                                  "flops_per_token": 2.0 * h * v,
                                                  "bf16_out_bytes": 2 * n * v,
                                                  "traffic": MEASURED_TRAFFIC.get(f"logprob_grad_{name}")}},
-        "gemms": "dL/dx = G @ w and dL/dw = G^T @ x, torch.mm (hipBLASLt)",
+        "gemms": "dL/dx = G @ w and dL/dw = G^T @ x, dsv41_head_dx_run and dsv41_head_dw_run",
     }
 
 

@@ -3930,7 +3930,7 @@ int plan(const dsv41_sampler_desc* d, Plan* pl, bool shard = false) {
   if (pl->lds > LDS_LIMIT)
     return fail(DSV41_E_UNSUPPORTED, "history length and vocabulary exceed the on-chip penalty tables");
   pl->defer = !shard && pl->mode == MODE_TOPK && d->rows > DEFER_MIN_ROWS;
-  // Batches of at least two rows per CU whose TOPP tables fit two workgroups per CU run
+  // Batches of more rows than CUs whose TOPP tables fit two workgroups per CU run
   // with 512 threads: a row's first read (memory) then overlaps another's mass pass (ALU).
   pl->topp_nt = pl->mode == MODE_TOPP && d->rows > 256 && 2 * pl->lds <= LDS_LIMIT ? 512 : TOPP_NT;
   // Deferred TOPK batches whose tables fit four 256-thread workgroups per CU (a quarter of
