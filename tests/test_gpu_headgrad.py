@@ -97,3 +97,22 @@ def test_refused_before_launch():
         assert lib.dsv41_head_dw_run(*bad, x.data_ptr(), x.stride(0), 8, 64, 64, w.data_ptr(), 72, stream) < 0
     assert lib.dsv41_head_dx_run(g.data_ptr(), g.stride(0), w.data_ptr(), w.stride(0), 8, 64, 60, x.data_ptr(), 0, None,
                                  0, stream) == m.E_UNSUPPORTED
+
+
+def test_vocabulary_above_the_offset_limit():
+    """A head whose whole row of logit gradients would pass the products' 32-bit block offsets."""
+    from dsv41_rocm.logprob import MAX_GRAD_COLUMNS, selected_log_probs
+
+    n, v, h = 3, 2 * MAX_GRAD_COLUMNS + 9, 8
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(n, h, generator=g, device="cuda").bfloat16().requires_grad_()
+    w = torch.randn(v, h, generator=g, device="cuda").bfloat16().requires_grad_()
+    t = torch.tensor([0, MAX_GRAD_COLUMNS, v - 1], device="cuda")
+    selected_log_probs(x, w, t)[0].sum().backward()
+    x64, w64 = (p.detach().double().requires_grad_() for p in (x, w))
+    torch.log_softmax(x64 @ w64.t(), -1).gather(1, t[:, None]).sum().backward()
+    # bf16 logit gradients and results: 2^-8 of the terms' magnitudes, which one term and the mean
+    # of the rows under the softmax (at most 1 by weight) make up
+    mag = w64.detach().abs()[t] + w64.detach().abs().max()
+    assert bool(((x.grad.double() - x64.grad).abs() <= 2.0 ** -7 * mag).all())
+    assert bool(((w.grad[t].double() - w64.grad[t]).abs() <= 2.0 ** -7 * (w64.grad[t].abs() + x64.detach().abs().sum(0))).all())

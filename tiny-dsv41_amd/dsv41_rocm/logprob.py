@@ -157,6 +157,9 @@ def logits_grad(hidden: torch.Tensor, weight: torch.Tensor, targets: torch.Tenso
 # = 1.06 GB); at 16384 tokens x 129280 rows it takes four ranges of 32768 rows.
 GRAD_BLOCK_BYTES = 1 << 30
 
+# Columns of one range: the products index a block of 256 rows of it with 32-bit byte offsets.
+MAX_GRAD_COLUMNS = 1 << 21
+
 # dL/dweight of fewer tokens than this is a write of the weights and little else, which the library
 # GEMM does faster (7168 x 129280: 32 tokens 0.46 ms against 0.53; 300 tokens 1.09 against 0.93).
 DW_MIN_TOKENS = 96
@@ -178,6 +181,7 @@ def selected_log_probs_backward(hidden, weight, targets, temperature, lse, entro
         return (torch.zeros_like(hidden) if need_hidden else None), (torch.zeros_like(weight) if need_weight else None)
     if vocab_chunk is None:
         vocab_chunk = max(256, GRAD_BLOCK_BYTES // max(1, 2 * n) // 256 * 256)
+    vocab_chunk = min(vocab_chunk, MAX_GRAD_COLUMNS)
     ranges = [(b, min(v, b + vocab_chunk)) for b in range(0, v, vocab_chunk)]
     # one range writes dx in bf16; several add up in fp32
     whole = len(ranges) == 1
