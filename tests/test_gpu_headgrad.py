@@ -116,3 +116,17 @@ def test_vocabulary_above_the_offset_limit():
     mag = w64.detach().abs()[t] + w64.detach().abs().max()
     assert bool(((x.grad.double() - x64.grad).abs() <= 2.0 ** -7 * mag).all())
     assert bool(((w.grad[t].double() - w64.grad[t]).abs() <= 2.0 ** -7 * (w64.grad[t].abs() + x64.detach().abs().sum(0))).all())
+
+
+@pytest.mark.parametrize("n", [0, 5, 100])
+def test_second_derivatives_are_refused(n):
+    """The kernels record no graph, on either side of the token count that picks them."""
+    from dsv41_rocm.logprob import selected_log_probs
+
+    x = torch.randn(n, 64, device="cuda").bfloat16().requires_grad_()
+    w = torch.randn(300, 64, device="cuda").bfloat16().requires_grad_()
+    lp = selected_log_probs(x, w, torch.zeros(n, dtype=torch.int64, device="cuda"))[0]
+    with pytest.raises(RuntimeError):
+        torch.autograd.grad(lp.sum(), (x, w), create_graph=True)
+    assert all(torch.isfinite(g).all() for g in torch.autograd.grad(
+        selected_log_probs(x, w, torch.zeros(n, dtype=torch.int64, device="cuda"))[0].sum(), (x, w)))

@@ -175,6 +175,8 @@ def selected_log_probs_backward(hidden, weight, targets, temperature, lse, entro
     ``dsv41_head_dw_run``.  Vocabulary ranges of ``vocab_chunk`` rows (default: as many as
     ``GRAD_BLOCK_BYTES`` allows) bound the logit gradient held at once.
     """
+    if need_weight and torch.is_grad_enabled() and hidden.requires_grad:
+        raise RuntimeError("the log-prob's backward does not support automatic differentiation (create_graph)")
     n, h = hidden.shape
     v = weight.shape[0]
     if n == 0:
