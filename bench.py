@@ -45,7 +45,7 @@ MEASURED_TRAFFIC = {
     "sampler_A": 4_951_450 + 318_464 + 79_872,  # sliced topk_kernel + merge_kernel (profiles/sampler_topk_A.md)
     "logprob_D": 46_112_195_686 + 1_048_576,
     "logprob_C": 7_592_285_070 + 1_245_184,  # fused_kernel + merge_kernel
-    "logprob_grad_D": 45_297_095_573 + 4_384_320_091,
+    "logprob_grad_D": 57_080_762_176 + 4_384_320_091,
 }
 
 
