@@ -39,6 +39,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "row_extent.h"
 
 namespace dsv41 {
 namespace sampler {
@@ -576,12 +577,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const void* base, uin
   // gfx9 raw buffer: stride 0, num_records = bytes; reads past it return 0
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
 }
-// The bytes of a row of V logits that its buffer serves.  The range check of a vector load goes
-// dword by dword, so every id of a row that ends inside a vector is read; an odd bf16 row's last
-// id shares its dword with one element past the row, which every user masks by V.
-template <typename TIn>
+// The bytes of a row of V logits that its buffer serves (VEC: read by vector loads).
+template <typename TIn, bool VEC>
 __device__ __forceinline__ uint32_t row_bytes(int V) {
-  return ((uint32_t)V * (uint32_t)sizeof(TIn) + 3u) & ~3u;
+  return row_extent(V, (int)sizeof(TIn), VEC);
 }
 
 // ------------------------------------------------------------ history tables
@@ -1076,7 +1075,7 @@ __global__ __launch_bounds__(PRE_NT) void full_slice_kernel(Params p) {
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int NC = n_chunks<G>(p.V), NE = n_mass_chunks(p.V);
   const int c1 = min((sl + 1) * p.slice_w, NC);
-  const __amdgpu_buffer_rsrc_t rs = row_rsrc(row_ptr<TIn>(p, row), row_bytes<TIn>(p.V));
+  const __amdgpu_buffer_rsrc_t rs = row_rsrc(row_ptr<TIn>(p, row), row_bytes<TIn, VEC>(p.V));
   float* oem = p.pre_em + (int64_t)row * NE;
   uint64_t* ow = p.pre_w + (int64_t)row * NE;
   int bad = 0;
@@ -1169,7 +1168,7 @@ __global__ __launch_bounds__(FULL_NT, sizeof(TIn) == 4 ? 8 : 1) void full_kernel
 
   const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const TIn* src = row_ptr<TIn>(p, row);
-  const __amdgpu_buffer_rsrc_t rs = row_rsrc(src, row_bytes<TIn>(p.V));
+  const __amdgpu_buffer_rsrc_t rs = row_rsrc(src, row_bytes<TIn, VEC>(p.V));
   constexpr int TILE = NT * G;
   int bad = 0;
   int U = 0;
@@ -2092,7 +2091,7 @@ __global__ __launch_bounds__(NTK) void topk_kernel(Params p) {
   HistIds<HR, IdT> hi;
   load_history<NT, HR>(p, row, hi);
   const TIn* src = row_ptr<TIn>(p, row);
-  const __amdgpu_buffer_rsrc_t rs = row_rsrc(src, row_bytes<TIn>(p.V));
+  const __amdgpu_buffer_rsrc_t rs = row_rsrc(src, row_bytes<TIn, VEC>(p.V));
   int bad = 0;
   int count = 0;            // candidates stored (uniform across the workgroup)
   float tau = NEG_INF;      // z of the top_k-th candidate once the buffer held top_k
@@ -2500,7 +2499,7 @@ __global__ __launch_bounds__(GEN_NT) void generic_kernel(Params p) {
     HistIds<HR> hi;
     load_history<NT, HR>(p, row, hi);
     const TIn* src = row_ptr<TIn>(p, row);
-    const __amdgpu_buffer_rsrc_t rs = row_rsrc(src, row_bytes<TIn>(p.V));
+    const __amdgpu_buffer_rsrc_t rs = row_rsrc(src, row_bytes<TIn, VEC>(p.V));
     float* zr = p.zbuf + (int64_t)row * p.V;
     constexpr int TILE = NT * G;
     int bad = 0;
@@ -2692,7 +2691,7 @@ __global__ __launch_bounds__(NT, 4) void topp_kernel(Params p) {
   HistIds<HR> hi;
   load_history<NT, HR>(p, row, hi);
   const TIn* src = row_ptr<TIn>(p, row);
-  const __amdgpu_buffer_rsrc_t rs = row_rsrc(src, row_bytes<TIn>(p.V));
+  const __amdgpu_buffer_rsrc_t rs = row_rsrc(src, row_bytes<TIn, VEC>(p.V));
   const int V = p.V;
 
   // ---- pass 1: maximum and its first index.  Its loads keep the default cache policy
@@ -3296,7 +3295,7 @@ __device__ __forceinline__ void slice_stream(const Params& p, int row, const His
   const int tid = threadIdx.x;
   HistIds<SM_HR> hi;
   load_history<NT, SM_HR>(p, row, hi);
-  const __amdgpu_buffer_rsrc_t rs = row_rsrc(row_ptr<TIn>(p, row), row_bytes<TIn>(p.V));
+  const __amdgpu_buffer_rsrc_t rs = row_rsrc(row_ptr<TIn>(p, row), row_bytes<TIn, VEC>(p.V));
   stream_row<TIn, G, NT, VEC, false, CPOL>(
       p, rs, h,
       [&]() {
@@ -3663,7 +3662,7 @@ __global__ __launch_bounds__(SM_FIN_NT) void small_topp_kernel(Params p) {
     if (p.has_pen) build_history<NT, SM_HR, true>(q, row, hi, h, m);
     landed(hi);
     if (wid == 0) {
-      const __amdgpu_buffer_rsrc_t rs = row_rsrc(row_ptr<TIn>(p, row), row_bytes<TIn>(V));
+      const __amdgpu_buffer_rsrc_t rs = row_rsrc(row_ptr<TIn>(p, row), row_bytes<TIn, false>(V));
       uint64_t ms[4], ls = 0;
       float zz[4];
 #pragma unroll
