@@ -2177,6 +2177,17 @@ __global__ __launch_bounds__(NTK) void topk_kernel(Params p) {
         float x[PF][G];
 #pragma unroll
         for (int k = 0; k < PF; ++k) unpack(R[k], x[k]);
+        // An odd bf16 row's last dword holds one element past the row: it reads zero too, or a head
+        // padded with -inf would send every row to the second look below.
+        if constexpr (VEC && sizeof(TIn) == 2) {
+          if ((p.V & 1) && t0 + PF >= nt) {
+#pragma unroll
+            for (int k = 0; k < PF; ++k)
+#pragma unroll
+              for (int j = 1; j < G; j += 2)
+                if ((t0 + k) * TILE + tid * G + j == p.V) x[k][j] = 0.0f;
+          }
+        }
         // the batch's first NT history slots, penalized exactly
         float zg = NEG_INF;
         uint32_t tg = 0;
