@@ -19,7 +19,7 @@ class _Word(threading.local):
     ptr = None
 
     def make(self):
-        self.host = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        self.host = torch.zeros(1, dtype=torch.int32, device="cpu", pin_memory=True)
         self.ptr = self.host.data_ptr()
 
 

@@ -76,7 +76,7 @@ def _upload(lengths, advantages, device):
     if advantages.device.type != "cpu":
         return torch.from_numpy(offsets).to(device), advantages.to(device).contiguous()
     cut = offsets.nbytes
-    host = torch.empty(cut + 4 * len(lengths), dtype=torch.uint8, pin_memory=True)
+    host = torch.empty(cut + 4 * len(lengths), dtype=torch.uint8, device="cpu", pin_memory=True)
     view = host.numpy()
     view[:cut] = offsets.view(np.uint8)
     view[cut:] = advantages.contiguous().numpy().view(np.uint8)
