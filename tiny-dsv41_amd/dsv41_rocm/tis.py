@@ -64,7 +64,7 @@ _CHECKS = (
 def _vector(value, like):
     """A detached float32 vector on like's device."""
     if type(value) is torch.Tensor and value.dtype == torch.float32 and value.device == like.device:
-        return value.detach() if value.requires_grad else value
+        return value.detach()  # (also where no gradient is required: a forward-mode tangent ends here too)
     return torch.as_tensor(value, dtype=torch.float32, device=like.device).detach()
 
 
