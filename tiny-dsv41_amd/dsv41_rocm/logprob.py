@@ -353,8 +353,11 @@ def token_log_probs(hidden: torch.Tensor, weight: torch.Tensor, targets: torch.T
     """Drop-in for model.py:679-684 (``_token_log_probs``): fp32 [B, T] with the selected
     targets' log-probs where ``mask`` is set and zeros elsewhere."""
     mask = mask.to(torch.bool)
-    if mask.shape != targets.shape or mask.shape != hidden.shape[:-1] or mask.device != hidden.device:
-        selected = hidden[mask]  # (shapes that only partly match, or raise as indexing does)
+    if (mask.ndim == 0 or mask.shape != targets.shape or mask.shape != hidden.shape[:-1]
+            or mask.device != hidden.device):
+        # a single token (whose place nonzero() gives an axis of its own), shapes that only partly
+        # match, or ones that raise as indexing does
+        selected = hidden[mask]
         if selected.shape[0] == 0:
             return torch.zeros(mask.shape, dtype=torch.float32, device=hidden.device)
         lp = selected_log_probs(selected, weight, targets[mask], temperature)[0]
