@@ -210,6 +210,24 @@ def selected_log_probs_backward(hidden, weight, targets, temperature, lse, entro
     return dx, dw
 
 
+class _FirstOrder(torch.autograd.Function):
+    """A gradient under create_graph: its value, and an error where it is differentiated again."""
+
+    @staticmethod
+    def forward(ctx, grad, *sources):
+        return grad.view_as(grad)
+
+    @staticmethod
+    def backward(ctx, *grads):
+        raise RuntimeError("the log-prob's gradients cannot be differentiated again")
+
+
+def first_order(grad, *sources):
+    """``grad``, which depends on ``sources`` through kernels that record no graph.  Under
+    create_graph a second differentiation raises instead of leaving its term out."""
+    return _FirstOrder.apply(grad, *sources) if grad is not None and torch.is_grad_enabled() else grad
+
+
 class _SelectedLogProbs(torch.autograd.Function):
     """Differentiable fused log-prob: forward = dsv41_logprob_run, backward =
     dsv41_logprob_grad_run + the two products.  The Token-TIS weight carries no gradient (the
@@ -231,7 +249,8 @@ class _SelectedLogProbs(torch.autograd.Function):
         dx, dw = selected_log_probs_backward(hidden, weight, targets, ctx.temperature, lse, ent, g_lp, g_ent,
                                              need_hidden=ctx.needs_input_grad[0],
                                              need_weight=ctx.needs_input_grad[1])
-        return dx, dw, None, None, None, None
+        sources = (hidden, weight, g_lp, g_ent)
+        return first_order(dx, *sources), first_order(dw, *sources), None, None, None, None
 
 
 def selected_log_probs(

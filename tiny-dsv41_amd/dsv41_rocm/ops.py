@@ -104,7 +104,8 @@ def _selected_log_probs_backward(ctx, g_lp, g_ent, g_ratio, g_lse):
         dx = dx.to(ctx.hidden_dtype)
     if dw is not None:
         dw = dw.to(ctx.weight_dtype)
-    return dx, dw, None, None, None, None
+    sources = (hidden, weight, g_lp, g_ent)
+    return _logprob.first_order(dx, *sources), _logprob.first_order(dw, *sources), None, None, None, None
 
 
 selected_log_probs_op.register_autograd(_selected_log_probs_backward, setup_context=_selected_log_probs_setup)
