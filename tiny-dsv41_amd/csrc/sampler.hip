@@ -69,13 +69,15 @@ constexpr int TOPP_NT = 1024;
 constexpr int TOPP_BINS = 4096;                // 32 octaves of (max - z) x 128 steps
 constexpr int TOPP_BIN_BASE = 100 << 7;        // octave 0 is [2^-27, 2^-26); smaller -> bin 0
 constexpr int TOPP_CAP = 4096;                 // list / boundary-bin tokens topp_kernel holds
-// Small top-p / min-p batches (small_*_kernel): at most so many rows (one workgroup per row is as
-// fast at 200 of top-p, 144 us both, and at 400 of min-p, 113 us), cut into so many slices in all
-// (top-p, whose bins cost every slice the same: 48 rows 74 us at 768, 79 at 1536, 87 at 3072).
+// Small top-p / min-p batches (small_*_kernel): at most so many rows (with one workgroup per row a
+// call of 200 rows of top-p took 144 us, as long as here), cut into so many slices in all
+// (top-p, whose bins cost every slice the same: 48 rows 74 us at 768, 79 at 1536, 87 at 3072;
+// both measured before the slices collected their tokens in LDS).
 constexpr int SMALL_TOPP_ROWS = 128, SMALL_MINP_ROWS = 256;
 constexpr int SMALL_TOPP_GRID = 768, SMALL_MINP_GRID = 1536;
 constexpr int SMALL_MIN_W = 2048;
 constexpr size_t SMALL_MAX_LDS = 64 * 1024;
+constexpr int SMALL_STAGE = 1024;  // tokens a slice collects in LDS before they go to the row's list
 static_assert(TOPP_CAP <= TOPP_BINS, "the boundary bin's tokens from the list go to the bins' space");
 constexpr size_t LDS_LIMIT = 160 * 1024;
 // Cache policy of the row streams: nt (non-temporal).  A pass reads each logit and history
@@ -3139,6 +3141,7 @@ struct MergeIn {
   const int32_t* status;  // [shards, rows]
   int shards, rows, stride;
   int take;  // keys used per list: min(stride, top_k), the size of the LDS buffer's shares
+  int leave = 0;  // status bits of rows that the launch behind redoes: they only pass their status on
 };
 
 __global__ __launch_bounds__(TOPK_NT) void merge_kernel(Params p, MergeIn in) {
@@ -3161,6 +3164,10 @@ __global__ __launch_bounds__(TOPK_NT) void merge_kernel(Params p, MergeIn in) {
       if (st) atomicOr(&m->status, st);
     }
     __syncthreads();
+    if (m->status & in.leave) {
+      if (tid == 0) p.out_status[row] = m->status;
+      return;
+    }
     if (tid == 0) {
       int a = 0;
       for (int s = 0; s < in.shards; ++s) {
@@ -3280,8 +3287,11 @@ __global__ __launch_bounds__(TOPK_NT) void merge_kernel(Params p, MergeIn in) {
 //           merge_kernel       the final selection over it
 // Every decision is the one topp_kernel or topk_kernel takes, on the same integers, so the ids and
 // kept sets are theirs.  Bound by the launches and their set-up at a few rows, by the masses and
-// bins at many.  A call of 48 bf16 rows with top-p 0.9 takes 134 us in topp_kernel and 72 here (8
-// fp32 rows 121 and 58, 128 rows 141 and 106); with min-p 0.05, 82 us in topk_kernel and 45 here.
+// bins at many.  Microseconds a checked call of bf16 rows of 151936 ids, one workgroup per row and
+// here, logits N(0, 1) - 1.1 log(rank) and N(0, 0.5): top-p 0.9, 8 rows 222 and 90, 238 and 106; 48
+// rows 225 and 112, 242 and 136; 128 rows 231 and 164, 245 and 196.  Min-p 0.05, 64 rows at T 0.6
+// 94 and 59; at T 1.5 124 and 71; 256 rows 96 and 84, 121 and 94.  From 8192 ids on, 1 to 128 (256)
+// rows, no such batch measured more than 1% slower than with one workgroup per row.
 constexpr int SM_NT = 256;
 constexpr int SM_HR = 4;
 
@@ -3338,6 +3348,36 @@ __device__ __forceinline__ void slice_stream(const Params& p, int row, const His
           hist(z, tok);
         }
       });
+}
+
+// The tokens a slice adds to its row's list: collected in LDS, then appended by one atomic on the
+// row's count.  (With an atomic of its own per token, waited for by its wave, small_keep_kernel took
+// 191 us on 64 rows of 151936 logits N(0, 2), now 44, and small_minp_kernel 52 on 128 rows of 32000,
+// now 8, and 739 where every token passes, now 65.)  A slice with more than the stage holds appends the rest one by one,
+// until the row's list is known to be full (count > TOPP_CAP: the row falls back).
+struct Stage {
+  uint64_t key[SMALL_STAGE];
+  int n, full, base;
+};
+__device__ __forceinline__ void stage_add(Stage* st, const Params& p, int row, uint64_t key) {
+  const int at = atomicAdd(&st->n, 1);
+  if (at < SMALL_STAGE) {
+    st->key[at] = key;
+  } else if (!*(volatile int*)&st->full) {
+    const int pos = atomicAdd(&p.sm_count[row], 1);
+    if (pos < TOPP_CAP) p.sm_list[(int64_t)row * TOPP_CAP + pos] = key;
+    else st->full = 1;
+  }
+}
+// Appends the stage; true if the row's list cannot hold it (all threads of the workgroup).
+__device__ __forceinline__ bool stage_flush(Stage* st, const Params& p, int row) {
+  __syncthreads();
+  const int n = min(st->n, SMALL_STAGE);
+  if (threadIdx.x == 0) st->base = n ? atomicAdd(&p.sm_count[row], n) : 0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += SM_NT)
+    if (st->base + i < TOPP_CAP) p.sm_list[(int64_t)row * TOPP_CAP + st->base + i] = st->key[i];
+  return st->full || st->base + n > TOPP_CAP;
 }
 
 // The row maximum over its slices' (every lane of every wave gets it).
@@ -3498,13 +3538,13 @@ __global__ __launch_bounds__(SM_NT) void small_keep_kernel(Params p) {
   const double dmax = (double)zmax;
   double es = 0.0;
   int nk = 0, bad = 0;
-  uint64_t* list = p.sm_list + (int64_t)row * TOPP_CAP;
-  auto boundary = [&](float z, int id) {
-    const int pos = atomicAdd(&p.sm_count[row], 1);
-    if (pos < TOPP_CAP) list[pos] = ckey(z, (uint32_t)id);
-  };
+  Stage* st = reinterpret_cast<Stage*>(smem + L.total);
+  auto boundary = [&](float z, int id) { stage_add(st, p, row, ckey(z, (uint32_t)id)); };
   slice_stream<TIn, VEC, 0>(
-      p, row, h, m, bad, []() {},
+      p, row, h, m, bad,
+      [&]() {
+        if (tid == 0) st->n = st->full = 0;
+      },
       [&](const float (&z)[4], int base, int) {
         // A percent of the ids pass: each round takes every lane's next one, so a wave runs the
         // 64-bit exp once or twice per tile and not once for each of a lane's four ids.
@@ -3546,6 +3586,7 @@ __global__ __launch_bounds__(SM_NT) void small_keep_kernel(Params p) {
           }
         }
       });
+  stage_flush(st, p, row);
   nk = block_sum_i<SM_NT>(nk, m);
   es = block_sum_d<SM_NT>(es, m);
   if (tid == 0) {
@@ -3725,28 +3766,28 @@ __global__ __launch_bounds__(SM_NT) void small_minp_kernel(Params p) {
   const Hist h = hist_tables(smem, L);
   const float zmax = small_row_max(p, row);
   const float bnd = minp_bound_f(zmax, p.lmin_f);  // at or below the exact bound
-  uint64_t* list = p.sm_list + (int64_t)row * TOPP_CAP;
+  Stage* st = reinterpret_cast<Stage*>(smem + L.total);
   int bad = 0;
   auto offer = [&](float z, int id) {
-    if (z > NEG_INF && z >= bnd && minp_ok(z, zmax, p)) {
-      const int pos = atomicAdd(&p.sm_count[row], 1);
-      if (pos < TOPP_CAP) list[pos] = ckey(z, (uint32_t)(v0 + id));
-      else atomicOr(&p.sm_status[row], ST_FALLBACK);
-    }
+    if (z > NEG_INF && z >= bnd && minp_ok(z, zmax, p)) stage_add(st, p, row, ckey(z, (uint32_t)(v0 + id)));
   };
   if (sl == 0 && threadIdx.x < 64) {  // the row's status so far, from its slices
-    int st = 0;
-    for (int s = threadIdx.x; s < p.n_slices; s += 64) st |= p.sm_part[row * p.n_slices + s].pad;
-    for (int o = 32; o > 0; o >>= 1) st |= __shfl_xor(st, o);
-    if (threadIdx.x == 0 && st) atomicOr(&p.sm_status[row], st);
+    int rs = 0;
+    for (int s = threadIdx.x; s < p.n_slices; s += 64) rs |= p.sm_part[row * p.n_slices + s].pad;
+    for (int o = 32; o > 0; o >>= 1) rs |= __shfl_xor(rs, o);
+    if (threadIdx.x == 0 && rs) atomicOr(&p.sm_status[row], rs);
   }
   slice_stream<TIn, VEC, 0>(
-      p, row, h, m, bad, []() {},
+      p, row, h, m, bad,
+      [&]() {
+        if (threadIdx.x == 0) st->n = st->full = 0;
+      },
       [&](const float (&z)[4], int base, int) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) offer(z[j], base + j);
       },
       [&](float z, int tok) { offer(z, tok); });
+  if (stage_flush(st, p, row) && threadIdx.x == 0) atomicOr(&p.sm_status[row], ST_FALLBACK);
 }
 
 // One thread per row of a full-vocabulary draw over slices: the row's maximum and total
@@ -4034,8 +4075,10 @@ int plan(const dsv41_sampler_desc* d, Plan* pl, bool shard = false) {
     if (Lg.total > LDS_LIMIT)
       return fail(DSV41_E_UNSUPPORTED, "history length and vocabulary exceed the on-chip penalty tables");
   }
-  // Top-p alone, or min-p without top-k, on few rows: slices of at least SMALL_MIN_W ids.  Their tables lie in the z rows of the fallback, which
-  // runs after them.
+  // Top-p alone, or min-p without top-k, on few rows: slices of at least SMALL_MIN_W ids.  Their
+  // tables lie in the z rows of the fallback, which runs after them: a row's list of 32 KiB and
+  // top-p's bins of 32 KiB fit its V floats from about 8300 (min-p) and 16600 ids (top-p) on, and
+  // shorter rows keep one workgroup each.
   pl->sm_slices = 0;
   const bool topp = pl->mode == MODE_TOPP;
   if (!shard && (topp || pl->internal_k) && d->rows <= (topp ? SMALL_TOPP_ROWS : SMALL_MINP_ROWS) && V >= 4 * SMALL_MIN_W) {
@@ -4060,7 +4103,7 @@ int plan(const dsv41_sampler_desc* d, Plan* pl, bool shard = false) {
     off += n * sizeof(int32_t);
     pl->sm_count = off;
     off += n * sizeof(int32_t);
-    if (S >= 2 && lds + (topp ? TOPP_BINS * sizeof(uint64_t) : 0) <= SMALL_MAX_LDS && fin <= LDS_LIMIT && off <= pl->workspace) {
+    if (S >= 2 && lds + (topp ? TOPP_BINS * sizeof(uint64_t) : sizeof(Stage)) <= SMALL_MAX_LDS && fin <= LDS_LIMIT && off <= pl->workspace) {
       pl->sm_slices = S;
       pl->slice_w = sw;
       pl->slice_words = words;
@@ -4306,18 +4349,20 @@ static int run_small(const dsv41_sampler_desc* d, const Plan& pl, const Params& 
   if (topp) {
     rc = launch(small_bins_kernel<TIn, VEC>, SM_NT, pl.sm_lds + TOPP_BINS * sizeof(uint64_t), grid, q, s);
     if (rc != DSV41_OK) return rc;
-    rc = launch(small_keep_kernel<TIn, VEC>, SM_NT, pl.sm_lds, grid, q, s);
+    rc = launch(small_keep_kernel<TIn, VEC>, SM_NT, pl.sm_lds + sizeof(Stage), grid, q, s);
     if (rc != DSV41_OK) return rc;
     q.ucap = pl.ucap;
     rc = launch(small_topp_kernel<TIn>, SM_FIN_NT, pl.sm_fin_lds, d->rows, q, s);
     return rc;
   }
-  rc = launch(small_minp_kernel<TIn, VEC>, SM_NT, pl.sm_lds, grid, q, s);
+  rc = launch(small_minp_kernel<TIn, VEC>, SM_NT, pl.sm_lds + sizeof(Stage), grid, q, s);
   if (rc != DSV41_OK) return rc;
   Params m = p;
   m.top_k = TOPP_CAP;
   m.topk_internal = 0;
-  MergeIn in{q.sm_list, q.sm_count, q.sm_status, 1, d->rows, TOPP_CAP, TOPP_CAP};
+  // (a row whose list overflowed goes to generic_kernel: sorting its 4096 keys first took 87 us of
+  // 64 rows' 1000)
+  MergeIn in{q.sm_list, q.sm_count, q.sm_status, 1, d->rows, TOPP_CAP, TOPP_CAP, ST_FALLBACK};
   DSV41_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(merge_kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_LIMIT));
   hipLaunchKernelGGL(merge_kernel, dim3(d->rows), dim3(TOPK_NT), merge_lds_bytes(TOPP_CAP, TOPP_CAP), s, m, in);
