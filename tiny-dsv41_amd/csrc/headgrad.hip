@@ -338,6 +338,8 @@ extern "C" int dsv41_head_dx_run(const void* g, int64_t gs, const void* w, int64
   const int r = out_mode == OUT_BF16 ? dx_ranges(n, v, h) : 1;
   if (r > 1 && (!workspace || workspace_bytes < (size_t)r * n * h * sizeof(float)))
     return fail(DSV41_E_WORKSPACE, "head gradient workspace is missing or too small");
+  if (r > 1 && (uintptr_t)workspace % 16)
+    return fail(DSV41_E_INVALID, "head gradient: the workspace must be 16-byte aligned");
   hipStream_t s = static_cast<hipStream_t>(stream);
   Params p{};
   p.w = static_cast<const uint16_t*>(w);
