@@ -549,7 +549,8 @@ int dsv41_logprob_grad_run(const dsv41_logprob_grad_desc* desc, void* stream /* 
  * dw[v, h] = sum_n g x with x [n, h], operands bf16, sums fp32.  Strides in elements, multiples of
  * 8; pointers 16-byte aligned, the workspace's too; h a multiple of 8.  out_mode: 0 writes dx in
  * bf16, 1 in fp32, 2 adds it to an fp32 dx (vocabulary ranges in turn); dx rows are h elements
- * apart.  The workspace serves mode 0.  They stand for the two GEMMs of nn.Linear's backward
+ * apart.  Mode 0 requires the workspace; modes 1 and 2 are faster with it where the tiles of dx
+ * leave CUs idle, and do without.  They stand for the two GEMMs of nn.Linear's backward
  * (distributed_grpo.py:352-375 over native_lora.py:120-122). */
 size_t dsv41_head_dx_workspace_bytes(int n, int v, int h);
 int dsv41_head_dx_run(const void* g, int64_t gs, const void* w, int64_t ws, int n, int v, int h, void* out,

@@ -284,8 +284,9 @@ __global__ __launch_bounds__(NT, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) v
   wait_loads<0>();  // no load to LDS outlives the loop
 }
 
-// bf16 sum over the contraction ranges, in their order.
-__global__ __launch_bounds__(256) void fold_kernel(const float4* part, int64_t step, int n, int64_t count, uint2* out) {
+// The contraction ranges' sums added up in their order: to bf16, to fp32, or onto what is there.
+template <int OUT>
+__global__ __launch_bounds__(256) void fold_kernel(const float4* part, int64_t step, int n, int64_t count, void* out) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= count) return;
   float4 s = part[i];
@@ -293,7 +294,16 @@ __global__ __launch_bounds__(256) void fold_kernel(const float4* part, int64_t s
     const float4 o = part[k * step + i];
     s = make_float4(s.x + o.x, s.y + o.y, s.z + o.z, s.w + o.w);
   }
-  out[i] = make_uint2(pack_bf16(s.x, s.y), pack_bf16(s.z, s.w));
+  if constexpr (OUT == OUT_BF16) {
+    static_cast<uint2*>(out)[i] = make_uint2(pack_bf16(s.x, s.y), pack_bf16(s.z, s.w));
+  } else {
+    float4* o = static_cast<float4*>(out) + i;
+    if constexpr (OUT == OUT_ADD) {
+      const float4 b = *o;
+      s = make_float4(b.x + s.x, b.y + s.y, b.z + s.z, b.w + s.w);
+    }
+    *o = s;
+  }
 }
 
 int check(const void* g, int64_t gs, const void* b, int64_t bs, const void* out, int n, int v, int h) {
@@ -309,12 +319,31 @@ int check(const void* g, int64_t gs, const void* b, int64_t bs, const void* out,
   return DSV41_OK;
 }
 
-// Contraction ranges of dx: its 256 x 256 tiles alone leave CUs idle below about 224 of them (2048
-// tokens x 7168), so the vocabulary is cut into ranges whose fp32 sums a second kernel adds.
+// Contraction ranges of dx.  Its 256 x 256 tiles alone leave CUs idle where they are few or fill
+// their last round badly, so the vocabulary is cut into ranges whose fp32 sums a second kernel adds
+// up: the count of the shortest estimate, rounds of workgroups as long as their stages and, with
+// more than one, the second kernel's passes over the sums (microseconds, measured; a range has at
+// least 8 stages and all sums at most 512 MiB).  Vocabulary x tokens x hidden, us in one range and
+// cut: 32768 x 4096 x 512 619 and 131 (8 ranges), 151936 x 4096 x 512 2823 and 526 (8), 64000 x
+// 2048 x 4608, 144 tiles, 1275 and 1017 (3); 129280 x 2048 x 7168, 224 tiles, 3022 and 3152 (2), left whole.
+constexpr double STAGE_US = 1.5, FILL_US = 5.0, FOLD_US = 5.0, FOLD_BYTES_PER_US = 4.5e6;
+constexpr size_t MAX_SUMS = (size_t)512 << 20;
+
 int dx_ranges(int n, int v, int h) {
-  const int tiles = (n + BN - 1) / BN * ((h + BM - 1) / BM), nk = (v + BK - 1) / BK;
-  if (tiles <= 0 || tiles > 3 * CU_COUNT / 4) return 1;
-  return std::max(1, std::min({CU_COUNT / tiles, nk / 8, 64}));
+  const int64_t tiles = (int64_t)((n + BN - 1) / BN) * ((h + BM - 1) / BM);
+  const int nk = (v + BK - 1) / BK;
+  const double sums = (double)n * h * sizeof(float);
+  int best = 1;
+  double best_us = 1e300;
+  for (int r = 1; r <= 64 && (r == 1 || (nk / r >= 8 && r * sums <= MAX_SUMS)); ++r) {
+    const double us = (double)((tiles * r + CU_COUNT - 1) / CU_COUNT) * ((nk + r - 1) / r * STAGE_US + FILL_US) +
+                      (r > 1 ? FOLD_US + 2 * r * sums / FOLD_BYTES_PER_US : 0.0);
+    if (us < 0.97 * best_us) {
+      best_us = us;
+      best = r;
+    }
+  }
+  return best;
 }
 
 }  // namespace headgrad
@@ -335,9 +364,11 @@ extern "C" int dsv41_head_dx_run(const void* g, int64_t gs, const void* w, int64
   if (rc != DSV41_OK) return rc;
   if (out_mode < OUT_BF16 || out_mode > OUT_ADD) return fail(DSV41_E_INVALID, "head gradient: unknown output mode");
   if (n == 0) return DSV41_OK;
-  const int r = out_mode == OUT_BF16 ? dx_ranges(n, v, h) : 1;
-  if (r > 1 && (!workspace || workspace_bytes < (size_t)r * n * h * sizeof(float)))
-    return fail(DSV41_E_WORKSPACE, "head gradient workspace is missing or too small");
+  int r = dx_ranges(n, v, h);
+  if (r > 1 && (!workspace || workspace_bytes < (size_t)r * n * h * sizeof(float))) {
+    if (out_mode == OUT_BF16) return fail(DSV41_E_WORKSPACE, "head gradient workspace is missing or too small");
+    r = 1;  // an fp32 dx takes its sums in place
+  }
   if (r > 1 && (uintptr_t)workspace % 16)
     return fail(DSV41_E_INVALID, "head gradient: the workspace must be 16-byte aligned");
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -362,8 +393,11 @@ extern "C" int dsv41_head_dx_run(const void* g, int64_t gs, const void* w, int64
   DSV41_HIP_CHECK(hipGetLastError());
   if (r > 1) {
     const int64_t count = (int64_t)n * h / 4;
-    hipLaunchKernelGGL(fold_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s,
-                       static_cast<const float4*>(workspace), count, r, count, static_cast<uint2*>(out));
+    const dim3 fgrid((unsigned)((count + 255) / 256));
+    const float4* part = static_cast<const float4*>(workspace);
+    if (out_mode == OUT_F32) hipLaunchKernelGGL(fold_kernel<OUT_F32>, fgrid, dim3(256), 0, s, part, count, r, count, out);
+    else if (out_mode == OUT_ADD) hipLaunchKernelGGL(fold_kernel<OUT_ADD>, fgrid, dim3(256), 0, s, part, count, r, count, out);
+    else hipLaunchKernelGGL(fold_kernel<OUT_BF16>, fgrid, dim3(256), 0, s, part, count, r, count, out);
     DSV41_HIP_CHECK(hipGetLastError());
   }
   return DSV41_OK;

@@ -195,7 +195,7 @@ def selected_log_probs_backward(hidden, weight, targets, temperature, lse, entro
         with torch.cuda.device(hidden.device):
             stream = torch.cuda.current_stream(hidden.device).cuda_stream
             if need_hidden:
-                ws_bytes = lib.dsv41_head_dx_workspace_bytes(n, e - b, h) if whole else 0
+                ws_bytes = lib.dsv41_head_dx_workspace_bytes(n, e - b, h)
                 ws = torch.empty(ws_bytes, dtype=torch.uint8, device=hidden.device) if ws_bytes else None
                 _lib.check(lib.dsv41_head_dx_run(g.data_ptr(), g.stride(0), weight[b:e].data_ptr(), weight.stride(0), n,
                                                  e - b, h, dx.data_ptr(), 0 if whole else (1 if b == 0 else 2),
