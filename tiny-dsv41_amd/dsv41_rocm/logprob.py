@@ -160,9 +160,42 @@ GRAD_BLOCK_BYTES = 1 << 30
 # Columns of one range: the products index a block of 256 rows of it with 32-bit byte offsets.
 MAX_GRAD_COLUMNS = 1 << 21
 
-# dL/dweight of fewer tokens than this is a write of the weights and little else, which the library
-# GEMM does faster (7168 x 129280: 32 tokens 0.46 ms against 0.53; 300 tokens 1.09 against 0.93).
-DW_MIN_TOKENS = 96
+# Where the library GEMM takes a product (as bf16 by bf16 to bf16, like nn.Linear's backward): dx of
+# few vocabulary columns, a contraction that the 256 x 256 tiles cut too coarsely (512 tokens x 512,
+# us: 4096 columns 18 and 27; 2048 x 4096: 4096 columns 64 and 74; at 8000 columns either, 16384 x
+# 2048 394 and 412, 2048 x 2048 81 and 70) ...
+DX_MIN_COLUMNS = 8192
+
+
+def _own_dw(n, columns, h):
+    """... and dw whose tiles do not fill the CUs once (2048 tokens, us: 16000 x 512, 126 tiles 41
+    and 53; 16000 x 1024, 252 tiles 67 and 59), or of so few tokens that it is a write of the
+    weights and little else (32768 x 2048, 160 tokens 44 and 51, 512 tokens 84 and 82; 129280 x
+    7168, 256 tokens 785 and 876, 512 tokens 1159 and 1162)."""
+    tiles = -(-columns // 256) * -(-h // 256)
+    return tiles >= 240 and n >= (256 if h <= 2048 else 512)
+
+
+def _dx(g, w, out, mode):
+    """out (mode 0: bf16, 1: fp32, 2: added to) = g @ w."""
+    lib = _lib.load()
+    n, columns, h = g.shape[0], g.shape[1], w.shape[1]
+    size = lib.dsv41_head_dx_workspace_bytes(n, columns, h)
+    ws = torch.empty(size, dtype=torch.uint8, device=g.device) if size else None
+    with torch.cuda.device(g.device):
+        stream = torch.cuda.current_stream(g.device).cuda_stream
+        rc = lib.dsv41_head_dx_run(g.data_ptr(), g.stride(0), w.data_ptr(), w.stride(0), n, columns, h, out.data_ptr(),
+                                   mode, None if ws is None else ws.data_ptr(), size, stream)
+    _lib.check(rc)
+
+
+def _dw(g, x, out):
+    """out = g.t() @ x in bf16."""
+    with torch.cuda.device(g.device):
+        stream = torch.cuda.current_stream(g.device).cuda_stream
+        rc = _lib.load().dsv41_head_dw_run(g.data_ptr(), g.stride(0), x.data_ptr(), x.stride(0), g.shape[0], g.shape[1],
+                                           x.shape[1], out.data_ptr(), out.stride(0), stream)
+    _lib.check(rc)
 
 
 def selected_log_probs_backward(hidden, weight, targets, temperature, lse, entropy, grad_logprob,
@@ -172,8 +205,9 @@ def selected_log_probs_backward(hidden, weight, targets, temperature, lse, entro
     The logit gradient comes from ``dsv41_logprob_grad_run`` (recomputed logits on the
     matrix cores, bf16 like the reference's ``lm_head`` output gradient); the two products
     with it, the reference's ``nn.Linear`` backward, are ``dsv41_head_dx_run`` and
-    ``dsv41_head_dw_run``.  Vocabulary ranges of ``vocab_chunk`` rows (default: as many as
-    ``GRAD_BLOCK_BYTES`` allows) bound the logit gradient held at once.
+    ``dsv41_head_dw_run``, or library GEMMs where their tiles are too few (``_own_dw``).
+    Vocabulary ranges of ``vocab_chunk`` rows (default: as many as ``GRAD_BLOCK_BYTES`` allows)
+    bound the logit gradient held at once.
     """
     if need_weight and torch.is_grad_enabled() and hidden.requires_grad:
         raise RuntimeError("the log-prob's backward does not support automatic differentiation (create_graph)")
@@ -187,24 +221,21 @@ def selected_log_probs_backward(hidden, weight, targets, temperature, lse, entro
     ranges = [(b, min(v, b + vocab_chunk)) for b in range(0, v, vocab_chunk)]
     # one range writes dx in bf16; several add up in fp32
     whole = len(ranges) == 1
-    dx = torch.empty(n, h, dtype=hidden.dtype if whole else torch.float32, device=hidden.device) if need_hidden else None
+    own_dx = not (whole and v < DX_MIN_COLUMNS)
+    dx = None
+    if need_hidden and own_dx:
+        dx = torch.empty(n, h, dtype=hidden.dtype if whole else torch.float32, device=hidden.device)
     dw = torch.empty_like(weight) if need_weight else None
-    lib = _lib.load()
     for b, e in ranges:
         g = logits_grad(hidden, weight, targets, temperature, lse, entropy, grad_logprob, grad_entropy, b, e)
-        with torch.cuda.device(hidden.device):
-            stream = torch.cuda.current_stream(hidden.device).cuda_stream
-            if need_hidden:
-                ws_bytes = lib.dsv41_head_dx_workspace_bytes(n, e - b, h)
-                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=hidden.device) if ws_bytes else None
-                _lib.check(lib.dsv41_head_dx_run(g.data_ptr(), g.stride(0), weight[b:e].data_ptr(), weight.stride(0), n,
-                                                 e - b, h, dx.data_ptr(), 0 if whole else (1 if b == 0 else 2),
-                                                 ws.data_ptr() if ws_bytes else None, ws_bytes, stream))
-            if need_weight and n < DW_MIN_TOKENS:
-                torch.mm(g.t(), hidden, out=dw[b:e])
-            elif need_weight:
-                _lib.check(lib.dsv41_head_dw_run(g.data_ptr(), g.stride(0), hidden.data_ptr(), hidden.stride(0), n,
-                                                 e - b, h, dw[b:e].data_ptr(), dw.stride(0), stream))
+        if need_hidden and own_dx:
+            _dx(g, weight[b:e], dx, 0 if whole else (1 if b == 0 else 2))
+        elif need_hidden:
+            dx = torch.mm(g, weight.detach())
+        if need_weight and _own_dw(n, e - b, h):
+            _dw(g, hidden, dw[b:e])
+        elif need_weight:
+            torch.mm(g.t(), hidden, out=dw[b:e])
     if dx is not None:
         dx = dx.to(hidden.dtype)
     return dx, dw
