@@ -115,8 +115,8 @@ __device__ __forceinline__ bool item_of(const Params& p, int b, int& tb, int& sp
   return true;
 }
 
-// e^(x ln 2): v_exp_f32 alone.  exp2f adds a rescue for results below 2^-126, which no sum
-// here can notice (the largest term of each is 1).
+// e^(x ln 2): v_exp_f32 alone.  exp2f adds a rescue for results below 2^-126, which the sums of
+// absorb cannot notice (the largest term of each is 1).
 __device__ __forceinline__ float exp2_raw(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // Folds one vocabulary block into the running (max z, sum e, sum e*z) of token column j.
@@ -179,7 +179,7 @@ __device__ __forceinline__ void grad_block(const Params& p, const floatx4 (&acc)
       for (int e = 0; e < 4; ++e) {
         const float a = acc[i][j][e];
         const float z = a * p.invT;
-        const float pr = exp2_raw(__builtin_fmaf(a, c1, -mb));
+        const float pr = exp2f(__builtin_fmaf(a, c1, -mb));  // (a result below 2^-126 is stored)
         const float onehot = (v0 + e == tl) ? 1.0f : 0.0f;
         const float g = glp * (onehot - pr) + gent * pr * (cent - z);
         gv[e] = g * p.invT;
