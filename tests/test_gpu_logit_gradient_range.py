@@ -8,11 +8,14 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n,v", [(3, 40), (300, 700)])
-def test_probabilities_below_the_smallest_normal(n, v):
+@pytest.mark.parametrize("every", [1, 7, 150])
+def test_probabilities_below_the_smallest_normal(n, v, every):
+    """In every token, or in some among others (the waves that have one take another exponential)."""
     from dsv41_rocm import logprob as L
 
     x = torch.zeros(n, 64, dtype=torch.bfloat16, device="cuda")
-    x[:, 0] = 1.0
+    x[:, 0] = 0.125
+    x[::every, 0] = 1.0
     w = torch.zeros(v, 64, dtype=torch.bfloat16, device="cuda")
     w[:, 0] = (-80.0 - torch.arange(v, device="cuda") % 13).bfloat16()  # 80 to 92 nats below
     w[0, 0] = 0.0
