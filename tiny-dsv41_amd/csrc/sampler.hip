@@ -40,6 +40,7 @@
 
 #include "common.h"
 #include "row_extent.h"
+#include "slice_rule.h"
 
 namespace dsv41 {
 namespace sampler {
@@ -69,8 +70,8 @@ constexpr int TOPP_NT = 1024;
 constexpr int TOPP_BINS = 4096;                // 32 octaves of (max - z) x 128 steps
 constexpr int TOPP_BIN_BASE = 100 << 7;        // octave 0 is [2^-27, 2^-26); smaller -> bin 0
 constexpr int TOPP_CAP = 4096;                 // list / boundary-bin tokens topp_kernel holds
-// Small top-p / min-p batches (small_*_kernel): at most so many rows (with one workgroup per row a
-// call of 200 rows of top-p took 144 us, as long as here), cut into so many slices in all
+// Small top-p / min-p batches (small_*_kernel; slice_rule.h): at most so many rows (with one
+// workgroup per row a call of 200 rows of top-p took 144 us, as long as here), cut into so many slices in all
 // (top-p, whose bins cost every slice the same: 48 rows 74 us at 768, 79 at 1536, 87 at 3072;
 // both measured before the slices collected their tokens in LDS).
 constexpr int SMALL_TOPP_ROWS = 128, SMALL_MINP_ROWS = 256;
@@ -3290,8 +3291,8 @@ __global__ __launch_bounds__(TOPK_NT) void merge_kernel(Params p, MergeIn in) {
 // bins at many.  Microseconds a checked call of bf16 rows of 151936 ids, one workgroup per row and
 // here, logits N(0, 1) - 1.1 log(rank) and N(0, 0.5): top-p 0.9, 8 rows 222 and 90, 238 and 106; 48
 // rows 225 and 112, 242 and 136; 128 rows 231 and 164, 245 and 196.  Min-p 0.05, 64 rows at T 0.6
-// 94 and 59; at T 1.5 124 and 71; 256 rows 96 and 84, 121 and 94.  From 8192 ids on, 1 to 128 (256)
-// rows, no such batch measured more than 1% slower than with one workgroup per row.
+// 94 and 59; at T 1.5 124 and 71; 256 rows 96 and 84, 121 and 94.  slice_rule.h says which batches go
+// this way, and why long histories keep one workgroup per row.
 constexpr int SM_NT = 256;
 constexpr int SM_HR = 4;
 
@@ -4080,6 +4081,7 @@ int plan(const dsv41_sampler_desc* d, Plan* pl, bool shard = false) {
   // top-p's bins of 32 KiB fit its V floats from about 8300 (min-p) and 16600 ids (top-p) on, and
   // shorter rows keep one workgroup each.
   pl->sm_slices = 0;
+  const int64_t hist = !pl->has_pen ? 0 : d->history_lens ? d->history_row_stride : d->hist_len;  // at most
   const bool topp = pl->mode == MODE_TOPP;
   if (!shard && (topp || pl->internal_k) && d->rows <= (topp ? SMALL_TOPP_ROWS : SMALL_MINP_ROWS) && V >= 4 * SMALL_MIN_W) {
     const int want = std::max(1, (topp ? SMALL_TOPP_GRID : SMALL_MINP_GRID) / d->rows);
@@ -4103,7 +4105,8 @@ int plan(const dsv41_sampler_desc* d, Plan* pl, bool shard = false) {
     off += n * sizeof(int32_t);
     pl->sm_count = off;
     off += n * sizeof(int32_t);
-    if (S >= 2 && lds + (topp ? TOPP_BINS * sizeof(uint64_t) : sizeof(Stage)) <= SMALL_MAX_LDS && fin <= LDS_LIMIT && off <= pl->workspace) {
+    if (S >= 2 && lds + (topp ? TOPP_BINS * sizeof(uint64_t) : sizeof(Stage)) <= SMALL_MAX_LDS && fin <= LDS_LIMIT &&
+        off <= pl->workspace && slices_pay(!topp, d->rows, S, V, pl->esize, hist)) {
       pl->sm_slices = S;
       pl->slice_w = sw;
       pl->slice_words = words;

@@ -1,0 +1,34 @@
+// slice_rule.h — where the sampler cuts a batch's rows over the GPU (sampler.hip): its kernels were
+// timed both ways, cut and with one workgroup per row, over the sizes named here.  Plain C++: the
+// host tests compile it.
+#pragma once
+
+#include <stdint.h>
+
+namespace dsv41 {
+
+// Every slice reads its row's whole history (`hist` ids at most; 0: no penalties) and builds a table
+// of its own part, so a batch whose histories are long against its rows is slower cut.  Times below
+// are cut / whole, checked calls, logits N(0, 1) - 1.1 log(rank).
+
+// Top-p alone and min-p without top-k in `slices` slices a row (small_*_kernel).  The histories cost
+// every CU its share of rows x slices of them, and a batch of more rows gains less.  Min-p reads
+// the logits twice where topk_kernel reads them once, which pays up to 125 MB of them (fp32 rows of
+// 129280: 200 rows 0.99, 256 rows 1.07).
+//   min-p, 129280 ids: 128 bf16 rows 0.72, with 2048 history ids 0.92, 4096 1.27; 64 rows 0.64, 2048
+//     0.77, 8192 1.50; 1 row 0.61, 8192 0.89, 16384 1.12.  32000 ids: 128 rows 0.86, 4096 1.35; 16
+//     rows 0.76, 2048 0.87, 8192 1.11.  12000 ids: 16 rows 0.91, 1024 0.90, 8192 1.19.
+//   top-p: 128 bf16 rows of 129280 0.72, 2048 0.83, 4096 1.05; 64 rows of 32000 0.85, 2048 0.95, 4096
+//     1.18; 1 row of 32000 0.78, 2048 0.86, 8192 1.17.
+// Up to 512 history ids no size was more than 8% slower cut (200 fp32 rows of 129280 with min-p,
+// 128 rows of 17000 with top-p).  Slices above 4096 ids hold larger tables, of which fewer fit a CU.
+inline bool slices_pay(bool min_p, int rows, int slices, int V, int esize, int64_t hist) {
+  if (min_p && (double)rows * V * esize > 125e6) return false;
+  if (hist <= 512) return true;
+  if (hist > 8192 || 7.8 * hist > V) return false;
+  const double share = rows * slices > 256 ? rows * slices / 256.0 : 1.0;
+  const double cost = (V > 4096 * (int64_t)slices ? 5.5 : 3.0) * share * hist;
+  return cost <= (V + (min_p ? 12000 : 0)) * (1.0 - rows / 256.0);
+}
+
+}  // namespace dsv41
