@@ -494,7 +494,8 @@ const char* dsv41_last_error(void);
  * all, S*top_k <= 4096) that
  * each leave their local top_k keys, a count and a status for a merge kernel on the
  * same stream; for a full-vocabulary batch that is spread over the GPU (at most 128 rows, and
- * bf16 ones of 257 to 448), rows*(12*ceil(vocab/256)+4*S) and alignment, which replays and the
+ * bf16 ones of 257 to 448, replays and the larger ones where their histories are short against
+ * the vocabulary), rows*(12*ceil(vocab/256)+4*S) and alignment, which replays and the
  * larger batches may do without (they then run one workgroup per row); none otherwise. */
 size_t dsv41_sampler_workspace_bytes(const dsv41_sampler_desc* desc);
 int dsv41_sampler_run(const dsv41_sampler_desc* desc, void* workspace, size_t workspace_bytes,
@@ -504,10 +505,10 @@ int dsv41_sampler_run(const dsv41_sampler_desc* desc, void* workspace, size_t wo
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  No
  * counterpart in the reference.  It runs dsv41_sampler_run's kernels with the workspace taken
  * from a static device array of DSV41_SAMPLER_STATIC_SCRATCH_BYTES per GPU (held by every GPU
- * the library runs on until the process ends) and calls no allocator.  A batch whose
- * dsv41_sampler_workspace_bytes exceeds that size returns DSV41_E_UNSUPPORTED before any
- * launch (4096 rows of top-k need 8.4 MB; the radix path's rows*vocab*4 bytes fit only small
- * batches).  The stream must belong to the current device; the first call on a device looks
+ * the library runs on until the process ends) and calls no allocator.  A batch that
+ * needs more than that size returns DSV41_E_UNSUPPORTED before any launch (4096 rows of top-k
+ * need 8.4 MB; the radix path's rows*vocab*4 bytes fit only small batches); one that may do
+ * without its workspace (above) runs without it then.  The stream must belong to the current device; the first call on a device looks
  * up the array's address there, so make it outside graph capture.  Every call on one GPU
  * shares that GPU's array: calls that overlap on one GPU (other streams, other threads)
  * race and must be serialised by the caller.  Nothing in the array needs clearing between

@@ -45,3 +45,30 @@ SLICES = [
 @pytest.mark.parametrize("args,way", SLICES)
 def test_top_p_and_min_p(tmp_path, args, way):
     assert _ask(tmp_path, f"slices_pay({args})") == way
+
+
+# replay, rows, vocabulary, history
+SPREAD = [
+    ("false, 128, 9000, 16384", "cut"),    # (draws of at most 128 rows always were)
+    ("true, 1, 151936, 0", "cut"),         # 0.68
+    ("true, 1, 151936, 16384", "cut"),     # (8192: 0.74)
+    ("true, 1, 9000, 0", "whole"),         # 1.10
+    ("true, 128, 129280, 1024", "cut"),    # 0.95
+    ("true, 128, 129280, 4096", "whole"),  # 1.11
+    ("true, 128, 32000, 2048", "whole"),   # 1.08
+    ("true, 64, 64000, 8192", "whole"),    # 1.13
+    ("false, 300, 2600, 0", "cut"),
+    ("false, 300, 129280, 0", "cut"),      # 0.85
+    ("false, 300, 9000, 1024", "cut"),     # 0.92
+    ("false, 300, 151936, 2048", "cut"),   # 0.91
+    ("false, 400, 151936, 4096", "whole"),  # 1.08
+    ("false, 448, 32000, 2048", "whole"),  # 1.16
+    ("false, 300, 9000, 8192", "whole"),   # 1.16
+    ("true, 448, 151936, 0", "cut"),       # 0.99
+    ("true, 300, 32000, 4096", "whole"),   # 1.15
+]
+
+
+@pytest.mark.parametrize("args,way", SPREAD)
+def test_full_vocabulary(tmp_path, args, way):
+    assert _ask(tmp_path, f"spread_pays({args})") == way

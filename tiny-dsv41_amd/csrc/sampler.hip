@@ -113,7 +113,7 @@ constexpr int DRAW_ARGMAX = 8;      // first largest logit without its log-prob:
 // Exact masses of the inverse-CDF draws are formed per chunk of MASS_CHUNK consecutive ids
 // of the row (or slice), against the chunk's own maximum.
 constexpr int MASS_CHUNK = 256;
-// FULL batches that are spread over the GPU (full_slice_kernel): few rows, and bf16 ones that one
+// FULL batches that are spread over the GPU (full_slice_kernel, where spread_pays): few rows, and bf16 ones that one
 // workgroup per row and CU takes in two rounds.  Measured, spread against whole rows (151936
 // ids, us a call): 128 rows fp32 52 and 60; 200 rows bf16 57 and 58, fp32 61 and 58; 256 rows
 // 71 and 60; 300 rows bf16 70 and 87, 400 rows 80 and 88; 500 rows fp32 109 and 90 (two
@@ -4043,8 +4043,10 @@ int plan(const dsv41_sampler_desc* d, Plan* pl, bool shard = false) {
   pl->pre_slices = 0;
   pl->pre_lds = 0;
   pl->required = pl->workspace;
+  const int64_t hist = !pl->has_pen ? 0 : d->history_lens ? d->history_row_stride : d->hist_len;  // at most
   if (!shard && pl->mode == MODE_FULL && !d->exponentials &&
-      (d->rows <= PRE_MAX_ROWS || (pl->esize == 2 && d->rows >= PRE_BF16_MIN && d->rows <= PRE_BF16_MAX))) {
+      (d->rows <= PRE_MAX_ROWS || (pl->esize == 2 && d->rows >= PRE_BF16_MIN && d->rows <= PRE_BF16_MAX)) &&
+      spread_pays(d->replay_ids != nullptr, d->rows, V, hist)) {
     const int G = pl->esize == 4 ? 4 : 8;  // the spread small batches take 4 fp32 logits per lane
     const int NC = (V + 64 * G - 1) / (64 * G), NE = n_mass_chunks(V);
     const int want = std::max(2, PRE_GRID / d->rows);
@@ -4081,7 +4083,6 @@ int plan(const dsv41_sampler_desc* d, Plan* pl, bool shard = false) {
   // top-p's bins of 32 KiB fit its V floats from about 8300 (min-p) and 16600 ids (top-p) on, and
   // shorter rows keep one workgroup each.
   pl->sm_slices = 0;
-  const int64_t hist = !pl->has_pen ? 0 : d->history_lens ? d->history_row_stride : d->hist_len;  // at most
   const bool topp = pl->mode == MODE_TOPP;
   if (!shard && (topp || pl->internal_k) && d->rows <= (topp ? SMALL_TOPP_ROWS : SMALL_MINP_ROWS) && V >= 4 * SMALL_MIN_W) {
     const int want = std::max(1, (topp ? SMALL_TOPP_GRID : SMALL_MINP_GRID) / d->rows);

@@ -11,6 +11,23 @@ namespace dsv41 {
 // of its own part, so a batch whose histories are long against its rows is slower cut.  Times below
 // are cut / whole, checked calls, logits N(0, 1) - 1.1 log(rank).
 
+// Full-vocabulary draws and replays (full_slice_kernel).
+//   draws, at most 128 rows: always cut.
+//   replays, at most 128 rows: 1 row of 151936 ids 0.68, of 32000 1.02, of 9000 1.10; 128 rows of
+//     129280 bf16 ids 0.90, with 1024 history ids 0.95, 4096 1.11; 64 rows of 64000 0.90, 2048 0.95,
+//     8192 1.13.
+//   257 to 448 bf16 rows, which gain less the more they fill a second round of CUs: 300 rows of
+//     129280 0.85, with 2048 history ids 0.93, 8192 1.15; 400 rows of 32000 1.02, 512 1.03, 2048 1.12;
+//     400 rows of 9000, where the finishing workgroups' histories are most of either, 0.98, 2048
+//     0.96, 8192 1.19.
+inline bool spread_pays(bool replay, int rows, int V, int64_t hist) {
+  if (rows > 128) {
+    const int64_t any = V < 10000 ? 4096 : V < 20000 ? 1024 : 512;
+    return hist <= any || hist * 6000 <= V * (int64_t)(460 - rows);
+  }
+  return !replay || (V >= 32000 && rows * hist + 40000 <= 2 * (int64_t)V);
+}
+
 // Top-p alone and min-p without top-k in `slices` slices a row (small_*_kernel).  The histories cost
 // every CU its share of rows x slices of them, and a batch of more rows gains less.  Min-p reads
 // the logits twice where topk_kernel reads them once, which pays up to 125 MB of them (fp32 rows of
