@@ -66,8 +66,9 @@ def test_logit_gradient_tile_edges(n, h, v):
 
 # the other cuts of a call into workgroups: the 512 x 128 tile (three blocks of tokens; one, with
 # the vocabulary shared evenly by rows), even row ranges of the 256 x 256 one, and two runs of
-# token blocks with ranges of their own (64 blocks of four ranges, the 65th of 129)
-ROUTES = [(331, 64, 40003), (100, 1024, 131071), (200, 1024, 60011), (16390, 128, 33001)]
+# token blocks with ranges of their own (64 blocks of four ranges, the 65th of 129; 256 blocks of one
+# range, the other two of 12).  test_logprob_cuts.py asserts that each takes its cut.
+ROUTES = [(331, 64, 40003), (100, 1024, 131071), (200, 1024, 60011), (16390, 128, 33001), (66000, 8, 3000)]
 
 
 @pytest.mark.parametrize("n,h,v", ROUTES)
