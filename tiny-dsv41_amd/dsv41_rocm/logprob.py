@@ -161,19 +161,24 @@ GRAD_BLOCK_BYTES = 1 << 30
 MAX_GRAD_COLUMNS = 1 << 21
 
 # Where the library GEMM takes a product (as bf16 by bf16 to bf16, like nn.Linear's backward): dx of
-# few vocabulary columns, a contraction that the 256 x 256 tiles cut too coarsely (512 tokens x 512,
-# us: 4096 columns 18 and 27; 2048 x 4096: 4096 columns 64 and 74; at 8000 columns either, 16384 x
-# 2048 394 and 412, 2048 x 2048 81 and 70) ...
-DX_MIN_COLUMNS = 8192
+# few vocabulary columns, a contraction that the 256 x 256 tiles cut too coarsely (hand-written /
+# library, 300 and 2048 tokens: 4096 columns x 512 1.34 and 1.23, x 2048 1.36 and 1.23, x 7168 1.10 and
+# 1.02; 6000 x 2048 0.82 and 0.89; 8000 x 2048 0.76 and 0.93) ...
+DX_MIN_COLUMNS = 6000
 
 
 def _own_dw(n, columns, h):
-    """... and dw whose tiles do not fill the CUs once (2048 tokens, us: 16000 x 512, 126 tiles 41
-    and 53; 16000 x 1024, 252 tiles 67 and 59), or of so few tokens that it is a write of the
-    weights and little else (32768 x 2048, 160 tokens 44 and 51, 512 tokens 84 and 82; 129280 x
-    7168, 256 tokens 785 and 876, 512 tokens 1159 and 1162)."""
+    """... and dw that is a write of the weights and little else, in the counts of tokens that the
+    library is fast at, multiples of 32 (hand-written / library, 7168 x 129280: 128 tokens 1.18, 256
+    1.13, 512 1.04, 1000 0.89, but 100 0.93, 300 0.86, 500 0.89; 2048 x 151936: 128 1.06, 256 0.90, 300
+    0.80), or whose tiles leave CUs idle for long (512 x 16000, 126 tiles: 300 tokens 0.88, 512 1.00,
+    2001 1.09, 4097 1.24; 512 x 20000, 158 tiles, 0.89, 1.01, 0.90 and 1.01).  Up to a round of tiles
+    no count is the library's (512 x 25600, 200 tiles: 128 tokens 0.76, 512 0.94).  Any count below 96
+    goes there."""
     tiles = -(-columns // 256) * -(-h // 256)
-    return tiles >= 240 and n >= (256 if h <= 2048 else 512)
+    if tiles < 150:
+        return 96 <= n < 448
+    return n >= (96 if n % 32 or tiles <= 256 else 256 if h <= 2048 else 512)
 
 
 def _dx(g, w, out, mode):
