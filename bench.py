@@ -43,9 +43,10 @@ MEASURED_TRAFFIC = {
     "sampler_B": 82_981_683 + 32_768,  # full_kernel (profiles/sampler_full_B.md)
     "sampler_E_full": 2_500_868_710 + 2_671_616,  # full_kernel (profiles/sampler_full_E_shape.md)
     "sampler_A": 4_951_450 + 318_464 + 79_872,  # sliced topk_kernel + merge_kernel (profiles/sampler_topk_A.md)
-    "logprob_D": 46_112_195_686 + 1_048_576,
-    "logprob_C": 7_592_285_070 + 1_245_184,  # fused_kernel + merge_kernel
-    "logprob_grad_D": 57_080_762_176 + 4_384_320_091,
+    "logprob_D": 46_635_629_205 + 1_599_658,  # fused_kernel + merge_kernel (profiles/logprob_fused_D.md)
+    "logprob_C": 7_630_545_177 + 1_258_291,  # the same (profiles/logprob_fused_C.md)
+    "logprob_grad_C": 8_032_774_464 + 2_489_329_744,  # fused_kernel<true> over the whole vocabulary
+    "logprob_grad_D": 59_468_017_152 + 4_236_254_752,  # the same (profiles/logprob_backward_D.md)
 }
 
 

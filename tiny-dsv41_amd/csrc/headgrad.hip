@@ -12,10 +12,10 @@
 // contraction x 128 columns per region (256 bytes a row), and its fragments come by
 // ds_read_b64_tr_b16, which hands every lane four elements down a column.  The rows' eight
 // 32-byte column groups are XOR-swizzled by (k & 3) | (k >> 3 & 1) << 2, which spreads the 16 rows
-// of a fragment read over all banks.  A library GEMM runs these two products at 0.87 and 0.95-1.05
-// PFLOP/s (2048 tokens, 7168 -> 129280, on one box: dx 4.33 ms, dw 3.49); here they take 2.91 and
-// 3.11 (1.31 and 1.22 PFLOP/s).  300 tokens: dx 0.86 -> 0.73 ms, dw 1.09 -> 0.93; 1000 tokens of 2048 ->
-// 151936: 0.87 -> 0.49 and 0.78 -> 0.60.  dw pays a store of its tile every 32 stages of 2048 tokens.
+// of a fragment read over all banks.  2048 tokens, 7168 -> 129280: dx 3.0 ms (1.26 PFLOP/s; a library
+// GEMM 4.36, 0.87), dw 3.22 (1.18; library 3.48, 1.09), 2.91 and 3.11 on another box; 300 tokens dx 723
+// us and 855, dw 932 and 1081; 1000 tokens of 2048 -> 151936 dx 509 and 859, dw 609 and 758.  dw pays a
+// store of its tile every 32 stages of 2048 tokens, and the fewer tokens, the more of it that store is.
 
 #include <algorithm>
 #include <type_traits>

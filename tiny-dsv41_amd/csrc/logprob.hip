@@ -9,8 +9,9 @@
 //
 // The contraction is computed transposed, C^T[v, n] = sum_k w[v, k] x[n, k], so that an
 // MFMA lane owns one token column and the per-token softmax state lives in registers.  A
-// workgroup owns BT = 256 tokens and sweeps a range of the vocabulary in BV = 256-row blocks
-// (each of its eight waves, two per SIMD, computes a 128 x 64 part); after each block the fp32
+// workgroup owns BT tokens and sweeps a range of the vocabulary in blocks of BV rows: the square
+// tile 256 x 256, the tall one 128 tokens x 512 rows (mfma_tile.h; plan_items chooses).  Each of its
+// eight waves, two per SIMD, computes a 128-row x 64-token part; after each block the fp32
 // accumulators update a running (max, sum e, sum e*z) per token.  A second kernel merges
 // the vocabulary ranges and computes the target logit as its own dot product.
 //
@@ -26,7 +27,7 @@
 // The two waves of a SIMD work in turns.  A stage has four phases, one per quarter of the
 // wave's tile (64 weight rows x 32 tokens over the whole stage: 16 MFMAs, 256 cycles), and a
 // phase two parts with a barrier behind each: the first reads the quarter's fragments and
-// issues two loads, the second multiplies.  Waves 4-7 start one barrier late, so on every SIMD
+// loads a region, the second multiplies.  Waves 4-7 start one barrier late, so on every SIMD
 // one wave multiplies while the other reads, and the matrix core passes from one to the other
 // at each barrier.  (With one barrier per stage and reads between the multiplies of both
 // waves, one wave ran ahead and idled at the barrier while the other finished alone below the
@@ -35,13 +36,15 @@
 // filled, 20.4 with the turns and 16x16x32; 8192 x 2048 -> 151936: 4.02, 3.65, 3.41 ms.)
 //
 // A quarter's rows are a region of the stage buffer (A0, A1, B0, B1: the halves of the weight
-// and of the token rows).  A region is reloaded as soon as its reads are over, not the stage:
+// and of the token rows), filled by each wave's LOADS_W or LOADS_X loads (square: 2 and 2, tall: 4
+// and 1).  A region is reloaded as soon as its reads are over, not the stage:
 //   read in phase        B0(s) end of 4s-1, A0(s) 4s, B1(s) 4s+1, A1(s) 4s+2 (read = its
 //                        fragments back before the multiplies of 4s, 4s, 4s+1, 4s+2 end)
 //   loaded for s+2 in    B0 4s+2, A0 4s+3, B1 4s+4, A1 4s+5
 // so every load is in flight for four to five phases (about 2500 cycles), and each wave waits
-// in every phase only until all but its last LOADS_AHEAD = 8 loads (four phases' worth) have
-// landed, one barrier before the first wave reads them.
+// in every phase only until all but its last AHEAD loads have landed, one barrier before the
+// first wave reads them.  AHEAD = 2 (LOADS_W + LOADS_X), 8 and 10, is what any four phases in a row
+// load: one of each region.
 //
 // Each 128-byte LDS row holds its eight 16-byte chunks XOR-swizzled by (row >> 1) & 7; with
 // that, a wave-wide 16-byte read of four chunks of 16 consecutive rows is free of bank
@@ -403,7 +406,7 @@ __global__ __launch_bounds__(NT, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) v
   wait_loads<0>();  // no load to LDS outlives the loop
 
   if constexpr (GRAD) return;
-  // combine the lane quarters (same tokens, interleaved rows), then the two vocab waves
+  // combine the lane quarters (same tokens, interleaved rows), then the waves along the vocabulary
 #pragma unroll
   for (int j = 0; j < WT; ++j)
 #pragma unroll
