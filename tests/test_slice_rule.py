@@ -17,28 +17,34 @@ def _ask(tmp_path, call):
     return subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.strip()
 
 
-# min-p, rows, slices, vocabulary, bytes a logit, history; cut / whole as timed
+# min-p, rows, slices, vocabulary, bytes a logit, history, depth (min-p); cut / whole as timed
 SLICES = [
-    ("true, 128, 12, 129280, 2, 0", "cut"),      # 0.72
-    ("true, 128, 12, 129280, 2, 2048", "cut"),   # 0.92
-    ("true, 128, 12, 129280, 2, 4096", "whole"),  # 1.27
-    ("true, 64, 22, 129280, 2, 8192", "whole"),  # 1.50
-    ("true, 1, 64, 129280, 4, 8192", "cut"),     # 0.92
-    ("true, 1, 64, 129280, 4, 16384", "whole"),  # 1.17
-    ("true, 256, 6, 64000, 4, 8192", "whole"),   # 2.84
-    ("true, 256, 6, 129280, 2, 64", "cut"),      # 0.99
-    ("true, 256, 6, 129280, 4, 0", "whole"),     # 1.07
-    ("true, 200, 7, 129280, 4, 0", "cut"),       # 0.99
-    ("true, 1, 6, 12000, 4, 16384", "whole"),    # 1.57
-    ("false, 128, 6, 32000, 2, 4096", "whole"),  # 1.38
-    ("false, 128, 6, 129280, 2, 2048", "cut"),   # 0.83
-    ("false, 4, 75, 151936, 4, 8192", "cut"),    # 0.61
-    ("false, 1, 16, 32000, 2, 8192", "whole"),   # 1.17
-    ("false, 1, 9, 17000, 2, 4096", "whole"),    # 1.10
-    ("false, 64, 12, 151936, 4, 4096", "cut"),   # 0.81
-    ("false, 64, 11, 32000, 2, 4096", "whole"),  # 1.18
-    ("true, 32, 43, 129280, 4, 4096", "cut"),    # 0.86
-    ("true, 64, 22, 151936, 2, 4096", "whole"),  # 1.12
+    ("true, 128, 12, 129280, 2, 0, 2.4", "cut"),      # 0.72
+    ("true, 128, 12, 129280, 2, 2048, 2.4", "cut"),   # 0.92
+    ("true, 128, 12, 129280, 2, 4096, 2.4", "whole"),  # 1.27
+    ("true, 64, 22, 129280, 2, 8192, 2.4", "whole"),  # 1.50
+    ("true, 1, 64, 129280, 4, 8192, 2.4", "cut"),     # 0.92
+    ("true, 1, 64, 129280, 4, 16384, 2.4", "whole"),  # 1.17
+    ("true, 256, 6, 64000, 4, 8192, 2.4", "whole"),   # 2.84
+    ("true, 256, 6, 129280, 2, 64, 2.4", "cut"),      # 0.99
+    ("true, 256, 6, 129280, 4, 0, 2.4", "whole"),     # 1.07
+    ("true, 200, 7, 129280, 4, 0, 2.4", "cut"),       # 0.99
+    ("true, 1, 6, 12000, 4, 16384, 2.4", "whole"),    # 1.57
+    ("false, 128, 6, 32000, 2, 4096, 2.4", "whole"),  # 1.38
+    ("false, 128, 6, 129280, 2, 2048, 2.4", "cut"),   # 0.83
+    ("false, 4, 75, 151936, 4, 8192, 2.4", "cut"),    # 0.61
+    ("false, 1, 16, 32000, 2, 8192, 2.4", "whole"),   # 1.17
+    ("false, 1, 9, 17000, 2, 4096, 2.4", "whole"),    # 1.10
+    ("false, 64, 12, 151936, 4, 4096, 2.4", "cut"),   # 0.81
+    ("false, 64, 11, 32000, 2, 4096, 2.4", "whole"),  # 1.18
+    ("true, 32, 43, 129280, 4, 4096, 2.4", "cut"),    # 0.86
+    ("true, 64, 22, 151936, 2, 4096, 2.4", "whole"),  # 1.12
+    ("true, 256, 6, 151936, 2, 0, 0.41", "whole"),  # 1.13
+    ("true, 256, 6, 151936, 2, 0, 1.8", "whole"),  # 1.00, with 300 history ids 1.16
+    ("true, 200, 7, 129280, 4, 300, 0.97", "whole"),  # 1.17
+    ("true, 160, 9, 129280, 2, 0, 0.97", "cut"),  # 0.91
+    ("true, 128, 12, 129280, 4, 0, 1.8", "cut"),  # 0.87
+    ("true, 256, 6, 129280, 2, 0, 4.7", "cut"),  # 0.84
 ]
 
 

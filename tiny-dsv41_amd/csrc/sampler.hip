@@ -4110,7 +4110,8 @@ int plan(const dsv41_sampler_desc* d, Plan* pl, bool shard = false) {
     pl->sm_count = off;
     off += n * sizeof(int32_t);
     if (S >= 2 && lds + (topp ? TOPP_BINS * sizeof(uint64_t) : sizeof(Stage)) <= SMALL_MAX_LDS && fin <= LDS_LIMIT &&
-        off <= pl->workspace && slices_pay(!topp, d->rows, S, V, pl->esize, hist)) {
+        off <= pl->workspace && slices_pay(!topp, d->rows, S, V, pl->esize, hist,
+                                             topp ? 0.0 : -(double)d->temperature * std::log((double)d->min_p))) {
       pl->sm_slices = S;
       pl->slice_w = sw;
       pl->slice_words = words;

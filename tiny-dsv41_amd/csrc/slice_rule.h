@@ -37,10 +37,19 @@ inline bool spread_pays(bool replay, int rows, int V, int64_t hist) {
 //     rows 0.76, 2048 0.87, 8192 1.11.  12000 ids: 16 rows 0.91, 1024 0.90, 8192 1.19.
 //   top-p: 128 bf16 rows of 129280 0.72, 2048 0.83, 4096 1.05; 64 rows of 32000 0.85, 2048 0.95, 4096
 //     1.18; 1 row of 32000 0.78, 2048 0.86, 8192 1.17.
+// Min-p is the faster whole the fewer tokens it keeps, those within `depth` = -T log(min_p) of the
+// largest logit, since topk_kernel then inserts few.  129280 ids, min-p 0.2 at T 0.6 (depth 0.97): 128
+// bf16 rows 0.84, 160 0.91, 200 0.99, 256 1.06, with 300 history ids 0.95, 1.04, 1.14, 1.22, fp32 0.97,
+// 1.11, 1.11, 1.20 (200 rows with history ids 1.17); min-p 0.05 (1.8): bf16 0.76, 0.84, 0.92, 0.98, fp32 0.87,
+// 1.05, 1.02; min-p 0.02 at T 1.2 (4.7): bf16 0.71, 0.73, 0.79, 0.84, fp32 0.75, 0.87, 0.88.
 // Up to 512 history ids no size was more than 8% slower cut (200 fp32 rows of 129280 with min-p,
 // 128 rows of 17000 with top-p).  Slices above 4096 ids hold larger tables, of which fewer fit a CU.
-inline bool slices_pay(bool min_p, int rows, int slices, int V, int esize, int64_t hist) {
-  if (min_p && (double)rows * V * esize > 125e6) return false;
+// depth: of no account for top-p.
+inline bool slices_pay(bool min_p, int rows, int slices, int V, int esize, int64_t hist, double depth) {
+  if (min_p) {
+    if ((double)rows * V * esize > 125e6) return false;
+    if (depth < 2 && rows > (esize == 4 ? 144 : 200) - (hist ? 32 : 0) - (depth < 1 ? 16 : 0)) return false;
+  }
   if (hist <= 512) return true;
   if (hist > 8192 || 7.8 * hist > V) return false;
   const double share = rows * slices > 256 ? rows * slices / 256.0 : 1.0;
